@@ -669,7 +669,7 @@ int collide_batch_status(fclx_context* ctx, const fclx_collide_batch_args* a, vo
     L.contact_pos = a->contact_pos;
     L.contact_normal = a->contact_normal;
     L.contact_depth = a->contact_depth;
-    e = launch_collide_plain(L, 2 * depth, s);
+    e = launch_collide_ordered(L, 2 * depth, s);
   } else if (a->engine == FCLX_ENGINE_BOOL) {
     if (nodes >= kFastMaxNodes || a->num_queries >= kFastMaxQueries) {
       L.cap = 1;  // min(count, 1)
@@ -684,6 +684,8 @@ int collide_batch_status(fclx_context* ctx, const fclx_collide_batch_args* a, vo
     // meshes and batches beyond the FAST engine's task encoding (node and
     // query index widths) take the plain kernel
     e = launch_collide_plain(L, 2 * depth, s);
+  } else if (a->engine == FCLX_ENGINE_FAST && a->num_max_contacts <= kOrderedCapMax) {
+    e = launch_collide_ordered(L, 2 * depth, s);
   } else if (a->engine == FCLX_ENGINE_FAST) {
     std::lock_guard<std::mutex> lock(ctx->ws_mu);
     e = engine_collide(ctx->ws, L, 2 * depth, s);
@@ -1403,7 +1405,7 @@ int collide_one(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_t 
       L.contact_normal = ctx->s_geo + 3 * ctx->s_pairs_cap;
       L.contact_depth = ctx->s_geo + 6 * ctx->s_pairs_cap;
     }
-    HIP_TRY(ctx, launch_collide_plain(L, depth_sum, s));
+    HIP_TRY(ctx, launch_collide_ordered(L, depth_sum, s));
     HIP_TRY(ctx, hipMemcpyAsync(&count, ctx->s_count, sizeof(count), hipMemcpyDeviceToHost, s));
     HIP_TRY(ctx, hipMemcpyAsync(st, ctx->s_stats, sizeof(st), hipMemcpyDeviceToHost, s));
     HIP_TRY(ctx, hipMemcpyAsync(&produced, ctx->s_num, sizeof(produced), hipMemcpyDeviceToHost,

@@ -9,17 +9,16 @@ struct EngineWorkspace;
 EngineWorkspace* engine_workspace_create();
 void engine_workspace_destroy(EngineWorkspace* ws);
 
-// Collide batch with the fast engine.  num_max_contacts <= kOrderedCapMax
-// runs the per-lane ordered traversal with FP32 culling; larger caps run the
-// breadth-first front expansion + persistent wavefront DFS, and re-run any
-// query whose contact count reaches the cap with the plain kernel so that
-// its truncated list is the reference's depth-first prefix.
+// Exhaustive collide batch (num_max_contacts > kOrderedCapMax; smaller caps
+// run launch_collide_ordered): breadth-first front expansion + persistent
+// wavefront DFS; any query whose contact count reaches the cap is cut to the
+// reference's depth-first prefix.
+hipError_t engine_collide(EngineWorkspace* ws, const CollideLaunch& L, int stack_need,
+                          hipStream_t s);
 // Booleans only: counts[q] = 1 when the query's pair collides, else 0; no
 // records or statistics.  Batches on different streams may overlap.
 hipError_t engine_anyhit_collide(EngineWorkspace* ws, const CollideLaunch& L, int stack_need,
                                  hipStream_t s);
-hipError_t engine_collide(EngineWorkspace* ws, const CollideLaunch& L, int stack_need,
-                          hipStream_t s);
 
 // Tunables of the exhaustive path, per context (defaults chosen by measurement).
 struct EngineTuning {

@@ -15,15 +15,13 @@
 //      Leaf candidates collect in an LDS queue and run 64 at a time, so the
 //      FP64 triangle tests execute with the wavefront converged.  Idle
 //      wavefronts refill from the front of phase 2;
-//   5. any query whose contact count reached the cap is re-run by the plain
-//      depth-first kernel and its records replaced (the reference stops at
-//      the cap-th contact in depth-first order).
+//   5. any query whose contact count reached the cap has its records cut to
+//      the reference's depth-first prefix: by path keys, or by a re-run in
+//      the reference's order.
 // Without early stop the set of BVTT nodes visited is order-independent, so
 // the contact set and the per-query test counts equal the reference's.
-//
-// Small caps (<= kOrderedCapMax, e.g. first contact): per-lane depth-first
-// traversal in the reference's order with FP32 culling, lanes refilling with
-// new queries as they finish.
+// (Small caps and contact geometry run in the reference's order:
+// kernels_ordered.hip.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,8 +29,7 @@
 #include <hipcub/hipcub.hpp>
 #include <vector>
 
-#include "device/cull32.h"
-#include "device/exact64.h"
+#include "device/query32.h"
 #include "engine.h"
 
 namespace fclx {
@@ -76,15 +73,6 @@ enum : int {
 };
 
 
-// FP64 relative pose of a query plus its meshes' triangle-major vertex
-// arrays: everything a triangle test needs, in one 128-B line.
-struct alignas(128) QueryXf64 {
-  double R[9];
-  double T[3];
-  const double* tv1;
-  const double* tv2;
-};
-
 // task = (query:22 | b1:21 | b2:21)
 __device__ __forceinline__ unsigned long long pack_task(int q, int b1, int b2) {
   return (static_cast<unsigned long long>(q) << 42) |
@@ -114,53 +102,6 @@ __device__ __forceinline__ unsigned long long wave_reserve(unsigned long long* c
   base = __shfl(base, leader);
   return base + static_cast<unsigned long long>(__popcll(mask & lanes_below())) * per_lane;
 }
-
-__device__ __forceinline__ bool query_ok(const MeshDev* meshes, int n, int i1, int i2) {
-  if (i1 < 0 || i2 < 0 || i1 >= n || i2 >= n) return false;
-  const MeshDev& a = meshes[i1];
-  const MeshDev& b = meshes[i2];
-  return a.num_bvs > 0 && b.num_bvs > 0 && a.bv_type == 0 && b.bv_type == 0;
-}
-
-__device__ __forceinline__ V3 vtx(const MeshDev& m, int i) {
-  const double* p = m.verts + 3 * static_cast<size_t>(i);
-  return v3(p[0], p[1], p[2]);
-}
-
-// R = R1^T R2, T = R1^T (t2 - t1)
-__device__ __forceinline__ void rel_pose64(const double* tf1, const double* tf2, double* R,
-                                           double* T) {
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      R[3 * i + j] = (tf1[i] * tf2[j] + tf1[3 + i] * tf2[3 + j]) + tf1[6 + i] * tf2[6 + j];
-  const V3 d = v3(tf2[9] - tf1[9], tf2[10] - tf1[10], tf2[11] - tf1[11]);
-  T[0] = dot(col(tf1, 0), d);
-  T[1] = dot(col(tf1, 1), d);
-  T[2] = dot(col(tf1, 2), d);
-}
-
-__device__ __forceinline__ void make_xf32(const double* R, const double* T, double cmax1,
-                                          double cmax2, QueryXf32& X) {
-#pragma unroll
-  for (int i = 0; i < 9; ++i) X.R[i] = static_cast<float>(R[i]);
-#pragma unroll
-  for (int i = 0; i < 3; ++i) X.T[i] = static_cast<float>(T[i]);
-  const double st = cmax1 + (fabs(T[0]) + fabs(T[1]) + fabs(T[2])) + cmax2;
-  // margin rounded up: the float conversion may round down by <= 2^-24
-  X.ms = static_cast<float>(static_cast<double>(kCullKS) * static_cast<double>(kCullU) * st *
-                            (1.0 + 1.0 / 1048576.0));
-}
-
-// Node and size arrays of a query's two meshes, read in parallel with the
-// query's transform so no mesh-descriptor load sits on the critical path.
-struct QueryPtr {
-  const ObbNode32* n1;
-  const ObbNode32* n2;
-  const double* s1;
-  const double* s2;
-};
 
 // Up to kSub + 1 ranges of tasks read as one sequence (the sub-buffers of a
 // deferred buffer and its dump region); consumers skip kNoTask entries.
@@ -230,7 +171,7 @@ __global__ void __launch_bounds__(kBlock) engine_setup(EngineArgs A) {
   bool valid = false;
   if (q < L.num_queries) {
     const int i1 = L.query_meshes[2 * q], i2 = L.query_meshes[2 * q + 1];
-    valid = query_ok(L.meshes, L.num_meshes, i1, i2);
+    valid = obbrss_query_ok(L.meshes, L.num_meshes, i1, i2);
     L.counts[q] = 0;
     A.qflag[q] = 0;
     if (L.bv_tests) L.bv_tests[q] = 0;
@@ -477,57 +418,8 @@ __global__ void __launch_bounds__(kBlock) engine_uncertain(EngineArgs A) {
 }
 
 // ----------------------------------------------- persistent depth-first
-// firstOverSecond's size comparison (bvh_collision_traversal_node-inl.h:
-// 77-89; OBBRSS::size = |OBB extents|^2, OBB-inl.h:206-209) from the FP32
-// extents already loaded with the nodes.  Each FP32 sum of squares is
-// within 5u (u = 2^-24) of the FP64 size, relative; outside a 50u band the
-// FP32 order is the FP64 order, inside it (ties included) and for sizes
-// near the FP32 underflow the FP64 sizes decide.  Saves the two scattered
-// 8-B size loads of almost every descent.
-__device__ __forceinline__ bool first_larger(const ObbNode32& n1, const ObbNode32& n2,
-                                             const double* s1, const double* s2) {
-  const float a = fmaf(n1.extent[2], n1.extent[2],
-                       fmaf(n1.extent[1], n1.extent[1], n1.extent[0] * n1.extent[0]));
-  const float b = fmaf(n2.extent[2], n2.extent[2],
-                       fmaf(n2.extent[1], n2.extent[1], n2.extent[0] * n2.extent[0]));
-  constexpr float kBand = 50.0f * 5.9604644775390625e-08f;
-  if (a > 1e-30f && b > 1e-30f) {
-    if (a > b * (1.0f + kBand)) return true;
-    if (a < b * (1.0f - kBand)) return false;
-  }
-  return *s1 > *s2;
-}
-
 // Outcome of the FP32 pass over one task.
 enum : int { kStepNone = 0, kStepPush = 1, kStepLeaf = 2, kStepUncertain = 3 };
-
-// A 64-B node record in four 16-B loads issued together (its child link
-// with the rest, not in a later load once the cull has passed).
-__device__ __forceinline__ ObbNode32 load_node32(const ObbNode32* p) {
-  const uint4* w = reinterpret_cast<const uint4*>(p);
-  const uint4 a = w[0], b = w[1], c = w[2], d = w[3];
-  ObbNode32 n;
-  uint4* o = reinterpret_cast<uint4*>(&n);
-  o[0] = a;
-  o[1] = b;
-  o[2] = c;
-  o[3] = d;
-  return n;
-}
-
-// The query's 64-B FP32 transform record, likewise in four 16-B loads.
-__device__ __forceinline__ QueryXf32 load_xf32(const QueryXf32* p) {
-  static_assert(sizeof(QueryXf32) == 64, "four 16-B words");
-  const uint4* w = reinterpret_cast<const uint4*>(p);
-  const uint4 a = w[0], b = w[1], c = w[2], d = w[3];
-  QueryXf32 x;
-  uint4* o = reinterpret_cast<uint4*>(&x);
-  o[0] = a;
-  o[1] = b;
-  o[2] = c;
-  o[3] = d;
-  return x;
-}
 
 // FP32-only BV test of task (q,b1,b2) and the descent rule; nothing FP64 is
 // inlined here, which keeps the depth-first kernel's register count low.
@@ -1240,7 +1132,7 @@ __global__ void __launch_bounds__(kBlock, kWavesPerSimd) engine_anyhit(CollideLa
     const int i1 = L.query_meshes[2 * qq], i2 = L.query_meshes[2 * qq + 1];
     if (L.bv_tests) L.bv_tests[qq] = 0;
     if (L.leaf_tests) L.leaf_tests[qq] = 0;
-    if (!query_ok(L.meshes, L.num_meshes, i1, i2)) {
+    if (!obbrss_query_ok(L.meshes, L.num_meshes, i1, i2)) {
       atomicOr(L.status, kStatusBadQuery);
       return false;
     }
@@ -1528,121 +1420,6 @@ __global__ void __launch_bounds__(kBlock, kWavesPerSimd) engine_anyhit(CollideLa
   }
 }
 
-// ---------------------------------------------- ordered, small caps
-template <int STACK>
-__global__ void __launch_bounds__(kBlock) ordered_collide(CollideLaunch L,
-                                                          unsigned long long* next) {
-  // per-lane state
-  int q = -1;
-  int count = 0;
-  long long bvt = 0, lft = 0;
-  int sp = 0, b1 = 0, b2 = 0;
-  bool overflow = false;
-  M3 R;
-  V3 T;
-  QueryXf32 X;
-  MeshDev m1{}, m2{};
-  int2 stack[STACK];
-  while (true) {
-    const bool need = q == -1;  // -2: the batch is exhausted for this lane
-    const unsigned long long nm = __ballot(need);
-    if (nm != 0) {
-      const int leader = __ffsll(static_cast<long long>(nm)) - 1;
-      unsigned long long base = 0;
-      if (lane_id() == leader) base = atomicAdd(next, static_cast<unsigned long long>(__popcll(nm)));
-      base = __shfl(base, leader);
-      if (need) {
-        const long long cand = static_cast<long long>(base + __popcll(nm & lanes_below()));
-        q = cand < L.num_queries ? static_cast<int>(cand) : -2;
-        if (q >= 0) {
-          const int i1 = L.query_meshes[2 * q], i2 = L.query_meshes[2 * q + 1];
-          count = 0;
-          bvt = lft = 0;
-          sp = 0;
-          b1 = b2 = 0;
-          if (!query_ok(L.meshes, L.num_meshes, i1, i2)) {
-            L.counts[q] = 0;
-            if (L.bv_tests) L.bv_tests[q] = 0;
-            if (L.leaf_tests) L.leaf_tests[q] = 0;
-            atomicOr(L.status, kStatusBadQuery);
-            q = -1;  // fetch again next round
-          } else {
-            m1 = L.meshes[i1];
-            m2 = L.meshes[i2];
-            double Rd[9], Td[3];
-            rel_pose64(L.tf1 + 12 * static_cast<size_t>(q), L.tf2 + 12 * static_cast<size_t>(q),
-                       Rd, Td);
-#pragma unroll
-            for (int k = 0; k < 9; ++k) R.m[k] = Rd[k];
-            T = v3(Td[0], Td[1], Td[2]);
-            make_xf32(Rd, Td, m1.cmax, m2.cmax, X);
-          }
-        }
-      }
-    }
-    if (__ballot(q != -2) == 0) break;
-    if (q < 0) continue;
-    // one BVTT node visit, as in the plain kernel
-    const int fc1 = m1.obb32[b1].first_child, fc2 = m2.obb32[b2].first_child;
-    ++bvt;
-    bool descend = false;
-    int r = obb_cull32(X, m1.obb32[b1], m2.obb32[b2]);
-    if (r == kCullUnsure) r = obb_overlap64(R, T, m1.obb64[b1], m2.obb64[b2]) ? 1 : 0;
-    if (r == kCullOverlap) {
-      if (fc1 < 0 && fc2 < 0) {
-        ++lft;
-        const int id1 = -(fc1 + 1), id2 = -(fc2 + 1);
-        const int32_t* t1 = m1.tris + 3 * static_cast<size_t>(id1);
-        const int32_t* t2 = m2.tris + 3 * static_cast<size_t>(id2);
-        if (tri_intersect64(vtx(m1, t1[0]), vtx(m1, t1[1]), vtx(m1, t1[2]), vtx(m2, t2[0]),
-                            vtx(m2, t2[1]), vtx(m2, t2[2]), R, T)) {
-          if (count < L.cap) {
-            const long long slot = static_cast<long long>(
-                atomicAdd(reinterpret_cast<unsigned long long*>(L.num_pairs), 1ULL));
-            if (slot < L.pair_capacity) {
-              L.pairs[3 * slot] = q;
-              L.pairs[3 * slot + 1] = id1;
-              L.pairs[3 * slot + 2] = id2;
-            } else if (L.pairs) {  // no buffer: counts only
-              atomicOr(L.status, kStatusPairOverflow);
-            }
-            ++count;
-          }
-        }
-      } else {
-        descend = true;
-      }
-    }
-    bool done = false;
-    if (descend) {
-      if (sp >= STACK) {
-        overflow = true;
-        done = true;
-      } else if ((fc2 < 0) || (fc1 >= 0 && (m1.size64[b1] > m2.size64[b2]))) {
-        stack[sp++] = make_int2(fc1 + 1, b2);
-        b1 = fc1;
-      } else {
-        stack[sp++] = make_int2(b1, fc2 + 1);
-        b2 = fc2;
-      }
-    } else if (sp == 0 || (count > 0 && count >= L.cap)) {
-      done = true;
-    } else {
-      const int2 e = stack[--sp];
-      b1 = e.x;
-      b2 = e.y;
-    }
-    if (done) {
-      L.counts[q] = count;
-      if (L.bv_tests) L.bv_tests[q] = bvt;
-      if (L.leaf_tests) L.leaf_tests[q] = lft;
-      if (overflow) atomicOr(L.status, kStatusStackOverflow);
-      overflow = false;
-      q = -1;
-    }
-  }
-}
-
 int device_cus() {
   static int cus = [] {
     int dev = 0, n = 0;
@@ -1726,11 +1503,9 @@ struct EngineWorkspace {
   double busy_sum = 0, busy_den = 0;
   EngineReport report{};
   EngineTuning tune{};
-  // work counters of the small-cap kernel: batches on different streams may
-  // run at once, so each launch takes the next slot of a ring (one cache
-  // line each) and waits for the slot's previous launch to end
-  static constexpr int kOrdSlots = 16;
-  // stack areas of the boolean kernel, a ring guarded like the counters
+  // stack areas of the boolean kernel: batches on different streams may run
+  // at once, so each launch takes an area of a ring and waits for the area's
+  // previous launch to end
   static constexpr int kAnySlots = 8;
   unsigned long long* any_stk[kAnySlots] = {};
   size_t any_cap[kAnySlots] = {};
@@ -1745,10 +1520,6 @@ struct EngineWorkspace {
   hipGraphExec_t all_graph = nullptr;
   std::vector<unsigned long long> all_key;
   hipStream_t cap_stream = nullptr;
-  unsigned long long* ord_ctr = nullptr;  // kOrdSlots x 16
-  hipEvent_t ord_ev[kOrdSlots] = {};
-  bool ord_used[kOrdSlots] = {};
-  int ord_next = 0;
 };
 
 EngineTuning& engine_tuning(EngineWorkspace* ws) { return ws->tune; }
@@ -1758,12 +1529,7 @@ EngineWorkspace* engine_workspace_create() {
   bool ok = hipMalloc(reinterpret_cast<void**>(&ws->counters),
                       kNumCounters * sizeof(unsigned long long)) == hipSuccess &&
             hipHostMalloc(reinterpret_cast<void**>(&ws->host_counters),
-                          kNumCounters * sizeof(unsigned long long)) == hipSuccess &&
-            hipMalloc(reinterpret_cast<void**>(&ws->ord_ctr),
-                      EngineWorkspace::kOrdSlots * 16 * sizeof(unsigned long long)) ==
-                hipSuccess;
-  for (int i = 0; ok && i < EngineWorkspace::kOrdSlots; ++i)
-    ok = hipEventCreateWithFlags(&ws->ord_ev[i], hipEventDisableTiming) == hipSuccess;
+                          kNumCounters * sizeof(unsigned long long)) == hipSuccess;
   for (int i = 0; ok && i < EngineWorkspace::kAnySlots; ++i)
     ok = hipEventCreateWithFlags(&ws->any_ev[i], hipEventDisableTiming) == hipSuccess;
   if (!ok) {
@@ -1788,11 +1554,6 @@ void engine_workspace_destroy(EngineWorkspace* ws) {
   (void)hipFree(ws->defer[0]);
   (void)hipFree(ws->defer[1]);
   if (ws->host_counters) (void)hipHostFree(ws->host_counters);
-  for (int i = 0; i < EngineWorkspace::kOrdSlots; ++i) {
-    if (ws->ord_used[i]) (void)hipEventSynchronize(ws->ord_ev[i]);
-    if (ws->ord_ev[i]) (void)hipEventDestroy(ws->ord_ev[i]);
-  }
-  (void)hipFree(ws->ord_ctr);
   for (int i = 0; i < EngineWorkspace::kAnySlots; ++i) {
     if (ws->any_used[i]) (void)hipEventSynchronize(ws->any_ev[i]);
     if (ws->any_ev[i]) (void)hipEventDestroy(ws->any_ev[i]);
@@ -1919,7 +1680,7 @@ unsigned leaf_grid(long long n) {
   return std::max(1u, std::min(grid_for(n), resident));
 }
 
-// Re-run the flagged queries with the plain depth-first kernel.
+// Re-run the flagged queries in the reference's order.
 hipError_t fixup_flagged(EngineWorkspace* ws, const CollideLaunch& L, int stack_need,
                          unsigned long long nflag, hipStream_t s) {
   const int nq = L.num_queries;
@@ -1960,7 +1721,7 @@ hipError_t fixup_flagged(EngineWorkspace* ws, const CollideLaunch& L, int stack_
     P.num_pairs = nrun;
     P.bv_tests = st;
     P.leaf_tests = st + nflag;
-    if ((e = launch_collide_plain(P, stack_need, s)) != hipSuccess) break;
+    if ((e = launch_collide_ordered(P, stack_need, s)) != hipSuccess) break;
   } while (false);
   if (e == hipSuccess) {
     // records produced by the fast engine
@@ -2451,28 +2212,9 @@ hipError_t engine_collide(EngineWorkspace* ws, const CollideLaunch& L, int stack
   if (!ws) return hipErrorInvalidValue;
   const int nq = L.num_queries;
   if (nq == 0) return hipSuccess;
-  const int cus = device_cus();
-  if (L.cap <= kOrderedCapMax) {
-    const int slot = ws->ord_next;
-    ws->ord_next = (slot + 1) % EngineWorkspace::kOrdSlots;
-    if (ws->ord_used[slot]) ENG_TRY(hipStreamWaitEvent(s, ws->ord_ev[slot], 0));
-    unsigned long long* ctr = ws->ord_ctr + 16 * slot;
-    set_u64<<<1, 1, 0, s>>>(ctr, 0);
-    const unsigned grid = static_cast<unsigned>(
-        std::min<long long>(grid_for(nq), static_cast<long long>(cus) * 8));
-    if (stack_need <= 64)
-      ordered_collide<64><<<grid, kBlock, 0, s>>>(L, ctr);
-    else if (stack_need <= 128)
-      ordered_collide<128><<<grid, kBlock, 0, s>>>(L, ctr);
-    else
-      ordered_collide<256><<<grid, kBlock, 0, s>>>(L, ctr);
-    ENG_TRY(hipGetLastError());
-    ENG_TRY(hipEventRecord(ws->ord_ev[slot], s));
-    ws->ord_used[slot] = true;
-    return hipSuccess;
-  }
   if (nq >= (1 << 22)) return hipErrorInvalidValue;  // task packing limit
   if (ws->tune.fast_persistent) return engine_persistent_collide(ws, L, stack_need, s);
+  const int cus = device_cus();
   const EngineTuning& tune = ws->tune;
   ENG_TRY(grow(ws->qx32, ws->qx32_cap, nq));
   ENG_TRY(grow(ws->qptr, ws->qptr_cap, nq));

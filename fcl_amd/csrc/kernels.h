@@ -112,6 +112,9 @@ hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& L, int waves, hipStr
 size_t mesh_shape_epa_lane_bytes();
 
 hipError_t launch_collide_plain(const CollideLaunch& L, int stack_need, hipStream_t s);
+// collide() in the reference's order by lane groups, any num_max_contacts,
+// with contact geometry and statistics on request (kernels_ordered.hip)
+hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStream_t s);
 
 // collide() with BVTT front lists: one lane per sequence of queries
 struct FrontLaunch {

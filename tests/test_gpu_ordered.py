@@ -1,0 +1,87 @@
+"""The lane-group collide kernel against the one-lane FP64 kernel (PLAIN, which
+the parity tests compare with the oracle): both group widths, list bounds,
+matrices that are no rotations, and contact mode; every answer, order and
+count equal."""
+import numpy as np
+import pytest
+import torch
+
+import fcl_amd as F
+from test_gpu_parity import _t, collide_gpu
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+@pytest.fixture(scope="module")
+def pair(ctx):
+    V, T = F.heightfield(24, 0.05, 5)
+    return [ctx.mesh(*F.icosphere(7, 0.15, 3)), ctx.mesh(F.scale_to_radius(V, 1.0), T)]
+
+
+def _same(ctx, qm, tf1, tf2, cap, stats):
+    a = collide_gpu(ctx, qm, tf1, tf2, cap, engine=F.ENGINE_PLAIN, stats=stats)
+    b = collide_gpu(ctx, qm, tf1, tf2, cap, engine=F.ENGINE_FAST, stats=stats)
+    assert a[0] == b[0] == 0 and a[5] == b[5]
+    assert np.array_equal(a[1], b[1])
+    assert a[2].keys() == b[2].keys() and all(np.array_equal(a[2][q], b[2][q]) for q in a[2])
+    assert np.array_equal(a[3], b[3]) and np.array_equal(a[4], b[4])
+    return a
+
+
+@pytest.mark.parametrize("n,cap,stats", [(65535, 1, False), (65536, 1, False), (65539, 1, False),
+                                         (65536, 1, True), (1, 64, True), (257, 2, True),
+                                         (300, 64, True), (300, 64, False)])
+def test_groups_match_the_one_lane_kernel(ctx, pair, n, cap, stats):
+    print("case: ordered groups n=%d cap=%d stats=%d" % (n, cap, stats), flush=True)
+    tf1, tf2 = F.poses(n, 0, 1.7, 0, 0x0D + n)
+    got = _same(ctx, np.tile(np.array(pair, np.int32), (n, 1)), tf1, tf2, cap, stats)
+    assert n == 1 or 0 < (got[1] > 0).mean() < 1
+
+
+def test_bad_queries_in_a_narrow_batch(ctx, pair):
+    n = 65537
+    print("case: ordered groups, bad queries n=%d" % n, flush=True)
+    tf1, tf2 = F.poses(n, 0, 1.7, 0, 0xBAD)
+    qm = np.tile(np.array(pair, np.int32), (n, 1))
+    bad = np.arange(0, n, 5)
+    qm[bad, 1] = 9999
+    rc, counts, per_q, _, _, _ = collide_gpu(ctx, qm, tf1, tf2, 1, engine=F.ENGINE_FAST,
+                                             stats=False)
+    assert rc != 0 and not counts[bad].any()
+    good = np.setdiff1d(np.arange(n), bad)
+    _, want, _, _, _, _ = collide_gpu(ctx, qm[good], tf1[good], tf2[good], 1, stats=False)
+    assert np.array_equal(counts[good], want)
+
+
+@pytest.mark.parametrize("scale", [1.0, 1.3, 40.0])
+def test_matrices_that_are_no_rotations(ctx, pair, scale):
+    """A scaled or sheared matrix is outside the FP32 cull's margin: the
+    single call and the batches answer as FP64 does."""
+    n = 60
+    print("case: ordered groups, scale %g" % scale, flush=True)
+    tf1, tf2 = F.poses(n, 0, 1.7, 0, 0x5CA1)
+    tf2[:, :9] *= scale
+    tf1[:, 1] += 0.2 * (scale - 1)
+    qm = np.tile(np.array(pair, np.int32), (n, 1))
+    want = _same(ctx, qm, tf1, tf2, 3, True)
+    for q in range(0, n, 7):
+        pairs, stats = ctx.collide(pair[0], tf1[q], pair[1], tf2[q], cap=3)
+        assert np.array_equal(pairs, want[2].get(q, np.zeros((0, 2))))
+        assert stats.tolist() == [want[3][q], want[4][q]]
+
+
+def test_a_full_list_of_hits(ctx):
+    """Two terrains through each other with a cap no query reaches: hits pile
+    up in the list behind open nodes."""
+    m = [ctx.mesh(*F.heightfield(20, 0.05, s)) for s in (9, 10)]
+    print("case: ordered groups, dense contacts", flush=True)
+    tf1, tf2 = F.poses(1, 0, 0.0, 0, 1)
+    tf2[0] = tf1[0]
+    n = 3
+    qm = np.tile(np.array(m, np.int32), (n, 1))
+    a = collide_gpu(ctx, qm, np.tile(tf1, (n, 1)), np.tile(tf2, (n, 1)), 100000, capacity=1 << 16)
+    pairs, stats = ctx.collide(m[0], tf1[0], m[1], tf2[0], cap=100000)
+    assert len(pairs) > 200 and np.array_equal(pairs, a[2][0])
+    assert stats.tolist() == [a[3][0], a[4][0]]
