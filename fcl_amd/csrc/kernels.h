@@ -80,7 +80,7 @@ struct ShapeLaunch {
   int32_t* status;
 };
 
-// Mesh (BVHModel<OBBRSS>) against a primitive shape, one query per lane.
+// Mesh (BVHModel<OBBRSS>) against a primitive shape.
 struct MeshShapeLaunch {
   const MeshDev* meshes;        // device table indexed by mesh id
   int32_t num_meshes;
@@ -103,8 +103,8 @@ struct MeshShapeLaunch {
   double* contact_depth;        // 1 per slot
   long long* stats;             // optional, 2 per query: BV tests, leaf tests
   int32_t* status;
-  int32_t leaf_share;           // percent of the live lanes waiting at leaves that starts a
-                                // leaf round (1..100; 0: 50, or 100 with contact)
+  int32_t leaf_share;           // percent of a wavefront's lanes with a leaf that starts a
+                                // leaf round (1..100; 0: 100)
   int32_t max_depth;            // deepest mesh of the context (levels)
 };
 // waves: register budget, 1..3 waves per SIMD

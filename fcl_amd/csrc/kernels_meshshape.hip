@@ -13,24 +13,22 @@
 //   (sphere_triangle-inl.h:138-230) for a sphere, GJK + EPA on the shape and
 //   the posed TriangleP for the others (gjk_solver_indep-inl.h:448-505).
 //
-// One query per lane.  A lane fits the shape's box (Jacobi eigenvectors of
-// the bound vertices' covariance), descends the mesh depth first with the
-// reference's child order and stops at num_max_contacts.  Without
-// enable_contact a GJK "inside" is the answer (EPA's status is never Failed
-// after it).  With it, GJK still decides the hit and the record's slot
-// (count, cap and order are GJK's), and EPA only supplies the slot's
-// contact: the lane queues GJK's final simplex with the slot, and a second
-// kernel runs EPA over the queue, each lane in a block of device memory of
-// its own, taking the next queued pair when its own ends.  (When the queue
-// for num_queries x num_max_contacts slots would not fit its budget, or
-// for meshes deeper than the LDS stack, the descending lane runs EPA
-// itself, in a grid sized to the EPA memory it holds.)
+// One lane per query fits the shape's box (Jacobi eigenvectors of the bound
+// vertices' covariance); then one wavefront per query descends the mesh in
+// the reference's order (device/ordered.h) and stops at num_max_contacts.
+// Without enable_contact a GJK "inside" is the answer (EPA's status is never
+// Failed after it).  With it, GJK still decides the hit and the record's
+// slot (count, cap and order are GJK's), and EPA only supplies the slot's
+// contact: committed hits are queued and a second kernel runs GJK and EPA
+// over the queue, each lane in a block of device memory of its own, taking
+// the next queued pair when its own ends.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
-#include "device/exact64.h"
 #include "device/fit64.h"
+#include "device/ordered.h"
+#include "device/query32.h"
 #include "device/shape64.h"
 #include "kernels.h"
 
@@ -39,18 +37,18 @@ namespace fclx {
 namespace {
 
 constexpr int kBlk = 256;
-constexpr int kMsStack = 64;  // pending right children in LDS: meshes up to this depth
-// deeper meshes (up to kMsDeepMax levels) keep the stack in device memory
+constexpr int kMsListCap = 512;    // entries of a query's list in LDS
+constexpr int kMsListDepth = 440;  // deepest mesh whose descent it holds beside a step
+// deeper meshes (up to kMsDeepMax levels) keep a stack in device memory
 constexpr int kMsDeepMax = 4096;
 constexpr int kMsDeepBlocksPerCu = 2;
 constexpr int kEpaBlocksPerCu = 2;
 constexpr size_t kEpaQueueBudget = size_t(4) << 30;  // bytes of queued EPA seeds at most
 
-// A hit whose contact EPA supplies: GJK's final simplex, the query, the
-// triangle and the record slot the contact goes to.
+// A hit whose contact EPA supplies: the query, the triangle and the record
+// slot the contact goes to.
 struct MsEpaSeed {
-  shp::D3 w[4], d[4];
-  int32_t q, rank, prim, pad;
+  int32_t q, prim;
   long long slot;
 };
 
@@ -356,57 +354,6 @@ __device__ __forceinline__ bool load_query(const MeshShapeLaunch& L, int q, shp:
   return false;
 }
 
-// Queries grouped by shape kind, so that a wavefront's lanes run the same
-// leaf test (the order of queries does not change any query's answer).
-// Keys: the five kinds, then 5 for a query whose shape id is out of range
-// (answered as a bad query by the main kernel).  ctr[0..5]: counts,
-// ctr[8..13]: placement cursors.
-constexpr int kKinds = 6;
-
-__device__ __forceinline__ int kind_of(const MeshShapeLaunch& L, int q) {
-  const int si = L.query_shapes[q];
-  if (si < 0 || si >= L.num_shapes) return kKinds - 1;
-  const int t = L.shapes[si].type;
-  return t >= 0 && t < kKinds - 1 ? t : kKinds - 1;
-}
-
-__global__ void ms_zero(int32_t* ctr) {
-  if (threadIdx.x < 16) ctr[threadIdx.x] = 0;
-}
-
-__global__ void __launch_bounds__(kBlk) ms_count(MeshShapeLaunch L, int32_t* ctr) {
-  __shared__ int cnt[kKinds];
-  if (threadIdx.x < kKinds) cnt[threadIdx.x] = 0;
-  __syncthreads();
-  const int i = blockIdx.x * kBlk + threadIdx.x;
-  if (i < L.num_queries) atomicAdd(&cnt[kind_of(L, i)], 1);
-  __syncthreads();
-  if (threadIdx.x < kKinds && cnt[threadIdx.x]) atomicAdd(&ctr[threadIdx.x], cnt[threadIdx.x]);
-}
-
-__global__ void __launch_bounds__(kBlk) ms_place(MeshShapeLaunch L, int32_t* ctr,
-                                                 int32_t* order) {
-  __shared__ int cnt[kKinds];
-  __shared__ int base[kKinds];
-  if (threadIdx.x < kKinds) cnt[threadIdx.x] = 0;
-  __syncthreads();
-  const int i = blockIdx.x * kBlk + threadIdx.x;
-  int key = 0, off = 0;
-  if (i < L.num_queries) {
-    key = kind_of(L, i);
-    off = atomicAdd(&cnt[key], 1);
-  }
-  __syncthreads();
-  if (threadIdx.x < kKinds) {
-    int start = 0;
-    for (int k = 0; k < static_cast<int>(threadIdx.x); ++k) start += ctr[k];
-    base[threadIdx.x] =
-        start + (cnt[threadIdx.x] ? atomicAdd(&ctr[8 + threadIdx.x], cnt[threadIdx.x]) : 0);
-  }
-  __syncthreads();
-  if (i < L.num_queries) order[base[key] + off] = i;
-}
-
 // The leaf test of one (shape, triangle) pair, kept out of line so that the
 // descent loop's registers are not sized for GJK and EPA.
 template <bool kContact>
@@ -449,26 +396,66 @@ __device__ __noinline__ bool leaf_test(const shp::Shape& s, const shp::Xf& T1, c
   return hit;
 }
 
-// The queued form of leaf_test<true>: a sphere's contact from the closed
-// form; for the other shapes GJK alone, its final simplex in g and
-// need_epa set on a hit.
-__device__ __noinline__ bool leaf_test_gjk(const shp::Shape& s, const shp::Xf& T1,
-                                           const shp::Xf& T2, const double* tv, double tol,
-                                           shp::Contact& c, shp::Gjk& g, bool& need_epa) {
-  need_epa = false;
-  if (s.type == shp::kSphere) {
+// One query of the group traversal, prepared by one lane.
+struct alignas(128) MsQuery {
+  double axis[9], to[3], ext[3];  // the shape's box in the world frame
+  int32_t valid;
+  int32_t unit;                   // the mesh's rotation and the box axes are unit vectors:
+                                  // the FP32 cull's margin holds
+};
+static_assert(sizeof(MsQuery) == 128, "one line per query");
+
+__global__ void __launch_bounds__(kBlk) meshshape_setup(MeshShapeLaunch L, MsQuery* out) {
+  const int q = blockIdx.x * kBlk + threadIdx.x;
+  if (q >= L.num_queries) return;
+  MsQuery r;
+  shp::Shape s;
+  r.valid = load_query(L, q, s, L.max_depth) ? 1 : 0;
+  r.unit = 0;
+  if (r.valid) {
+    shape_obb(s, shp::xf_load(L.tf2 + 12 * static_cast<size_t>(q)), r.axis, r.to, r.ext);
+    const double* R = L.tf1 + 12 * static_cast<size_t>(q);
+    bool unit = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      unit = unit && sq(col(R, k)) < 1.0001 && sq(v3(R[3 * k], R[3 * k + 1], R[3 * k + 2])) < 1.0001 &&
+             sq(col(r.axis, k)) < 1.0001;
+    r.unit = unit ? 1 : 0;
+  } else {
+    L.counts[q] = 0;
+    if (L.stats) {
+      L.stats[2 * q] = 0;
+      L.stats[2 * q + 1] = 0;
+    }
+    atomicOr(L.status, kStatusBadQuery);
+  }
+  out[q] = r;
+}
+
+// A group's query in LDS.
+struct MsWave {
+  shp::Shape s;
+  shp::Xf T1, T2;
+  MsQuery m;
+  QueryXf32 x32;   // the mesh's pose, with the cull's margin
+  ObbNode32 box32; // the shape's box
+  const ObbNode32* n32;
+  const ObbNode64* n64;
+  const double* tris;
+};
+
+// The leaf test's answer alone: a sphere by the closed form, the other
+// shapes by GJK.  Out of line, so that the traversal's registers are not
+// sized for it.
+__device__ __forceinline__ bool leaf_inside(const MsWave& w, const double* tv, double tol) {
+  if (w.s.type == shp::kSphere) {
     D3 P[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) P[k] = shp::apply(T1, mk(tv[3 * k], tv[3 * k + 1], tv[3 * k + 2]));
+    for (int k = 0; k < 3; ++k)
+      P[k] = shp::apply(w.T1, mk(tv[3 * k], tv[3 * k + 1], tv[3 * k + 2]));
     D3 p, n;
     double d;
-    const bool hit = sphere_triangle(s.dims[0], T2.t, P[0], P[1], P[2], p, d, n);
-    if (hit) {
-      c.pos = p;
-      c.normal = shp::neg(n);
-      c.depth = d;
-    }
-    return hit;
+    return sphere_triangle(w.s.dims[0], w.T2.t, P[0], P[1], P[2], p, d, n);
   }
   shp::Shape tri;
   tri.type = shp::kTriangle;
@@ -476,10 +463,176 @@ __device__ __noinline__ bool leaf_test_gjk(const shp::Shape& s, const shp::Xf& T
   tri.dims[0] = tri.dims[1] = tri.dims[2] = 0;
   tri.verts = tv;
   shp::MDiff m;
-  shp::make_mdiff(s, T2, tri, T1, m);
-  const bool hit = shp::gjk_evaluate(g, m, tol) == shp::kGjkInside;
-  need_epa = hit;
-  return hit;
+  shp::make_mdiff(w.s, w.T2, tri, w.T1, m);
+  shp::Gjk g;
+  return shp::gjk_evaluate(g, m, tol) == shp::kGjkInside;
+}
+
+// collide(mesh, shape) in the reference's order (device/ordered.h), one
+// wavefront per query: FP32 certified culls of the mesh's nodes against the
+// shape's box (FP64 where unsure), leaf tests once leaf_min leaf entries
+// have gathered or nothing else is left to test.  With contacts, a committed
+// hit takes its record slot; spheres write their contact at once, the others
+// are queued for EPA.
+//
+// Bound: GJK, about 75 us for a round of up to 64 at two wavefronts per SIMD
+// (two thirds of the kernel), whatever the number of lanes in it; so a
+// round waits for a full wavefront of leaves (leaf_min 64; 100,000 links
+// around 20,480 triangles, 258 nodes and 79 leaves on average and up to
+// 20,713 and 9,888: 11.1 ms, at 32 14.1 ms, at 16 19.4 ms).  One lane per
+// query, as before, took 330-460 ms for this batch, the time of its longest
+// query; 200,000 links that nearly all collide at once 8.3 ms, now 7.3.
+// Quarter wavefronts are faster for the latter (4.2 ms) and slower for the
+// former (28 ms).
+template <bool kStats, bool kContact, int kWaves>
+__global__ void __launch_bounds__(64, kWaves) meshshape_ordered(MeshShapeLaunch L,
+                                                                const MsQuery* queries, int margin,
+                                                                int leaf_min, MsEpaSeed* seeds,
+                                                                unsigned long long* nseed) {
+  constexpr int G = 64, kCap = kMsListCap;
+  __shared__ OrderedList<kCap, kStats> S;
+  __shared__ MsWave w;
+  const LaneGroup<G> g;
+  const size_t q = blockIdx.x;
+  if (queries[q].valid == 0) return;
+  OrdTotals T;
+  if (g.lane == 0) {
+    const MeshDev& M = L.meshes[L.query_meshes[q]];
+    (void)load_query(L, static_cast<int>(q), w.s, L.max_depth);
+    w.T1 = shp::xf_load(L.tf1 + 12 * q);
+    w.T2 = shp::xf_load(L.tf2 + 12 * q);
+    const MsQuery m = queries[q];
+    w.m = m;
+    QueryXf32 X;
+    make_xf32(w.T1.R, w.T1.t.v, (fabs(m.to[0]) + fabs(m.to[1])) + fabs(m.to[2]), M.cmax, X);
+    if (!m.unit) X.ms = INFINITY;  // every test is left to FP64
+    X.m1 = X.m2 = 0;
+    X.valid = 1;
+    w.x32 = X;
+    ObbNode32 b;
+#pragma unroll
+    for (int k = 0; k < 9; ++k) b.axis[k] = static_cast<float>(m.axis[k]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      b.to[k] = static_cast<float>(m.to[k]);
+      b.extent[k] = static_cast<float>(m.ext[k]);
+    }
+    b.first_child = 0;
+    w.box32 = b;
+    w.n32 = M.obb32;
+    w.n64 = M.obb64;
+    w.tris = M.tri_verts;
+    S.e[0] = ord_pack(kOrdNode, 0, 0);
+    if constexpr (kStats) S.acc[0] = make_uint2(0u, 0u);
+  }
+  T.sp = 1;
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  while (T.sp > 0) {
+    const int n = ord_window<G, kCap>(T.sp, margin);
+    const bool on = g.lane < n;
+    unsigned long long e = 0;
+    uint2 acc = make_uint2(0u, 0u);
+    if (on) {
+      e = S.e[T.sp - 1 - g.lane];
+      if constexpr (kStats) acc = S.acc[T.sp - 1 - g.lane];
+    }
+    const int kind = ord_kind(e), id = ord_a(e);
+    const bool node = on && kind == kOrdNode, leaf = on && kind == kOrdLeaf;
+    OrdOutcome r;
+    if (on && kind >= kOrdHit) {
+      r.nout = 1;
+      r.o0 = e;
+      r.hit = true;
+      r.n = 1;
+    }
+    const unsigned long long lm = __ballot(leaf);
+    const bool test_leaves = lm != 0 && (__popcll(lm) >= leaf_min || __ballot(node) == 0);
+    if (node) {
+      const ObbNode32 nd = load_node32(w.n32 + id);
+      r.bv = 1;
+      int c = obb_cull32(w.x32, w.box32, nd);
+      if (c == kCullUnsure) {
+        const ObbNode64& n64 = w.n64[id];
+        M3 R0;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) R0.m[i] = w.T1.R[i];
+        double B[9], Tr[3];
+        box_relative(R0, v3(w.T1.t.v[0], w.T1.t.v[1], w.T1.t.v[2]), w.m.axis, w.m.to, n64.axis,
+                     n64.to, B, Tr);
+        c = obb_disjoint64(B, Tr, w.m.ext, n64.extent) ? kCullDisjoint : kCullOverlap;
+      }
+      if (c == kCullOverlap) {
+        const int fc = nd.first_child;
+        if (fc >= 0) {
+          r.nout = 2;
+          r.o0 = ord_pack(kOrdNode, fc, 0);
+          r.o1 = ord_pack(kOrdNode, fc + 1, 0);
+        } else {
+          r.nout = 1;
+          r.o0 = ord_pack(kOrdLeaf, -(fc + 1), 0);
+        }
+      }
+    } else if (leaf) {
+      if (test_leaves) {
+        r.leaf = 1;
+        if (leaf_inside(w, w.tris + static_cast<size_t>(id) * kTriVertsStride, L.tol)) {
+          r.nout = 1;
+          r.hit = true;
+          r.n = 1;
+          r.o0 = ord_pack(kOrdHit + 1, id, 0);
+        }
+      } else {
+        r.nout = 1;
+        r.o0 = e;
+      }
+    }
+    ord_settle<G, kCap, kStats>(g, S, T, r, acc, n, L.cap, [&](bool mine, int take, int before,
+                                                               int total) {
+      (void)total;
+      const bool store = mine && take > 0;
+      const size_t slot = q * L.cap + T.count + before;
+      const int prim = ord_a(r.o0);
+      if (store && L.prims) L.prims[slot] = prim;
+      if constexpr (kContact) {
+        const bool sphere = w.s.type == shp::kSphere;
+        const unsigned long long em = __ballot(store && !sphere);
+        if (em != 0) {  // one reservation for the wavefront
+          const int leader = __ffsll(static_cast<long long>(em)) - 1;
+          unsigned long long b = 0;
+          if (static_cast<int>(__lane_id()) == leader)
+            b = atomicAdd(nseed, static_cast<unsigned long long>(__popcll(em)));
+          b = __shfl(b, leader);
+          if (store && !sphere)
+            seeds[b + __popcll(em & ((1ULL << __lane_id()) - 1ULL))] =
+                MsEpaSeed{static_cast<int32_t>(q), prim, static_cast<long long>(slot)};
+        }
+        if (store && sphere) {
+          const double* tv = w.tris + static_cast<size_t>(prim) * kTriVertsStride;
+          D3 P[3];
+#pragma unroll
+          for (int k = 0; k < 3; ++k)
+            P[k] = shp::apply(w.T1, mk(tv[3 * k], tv[3 * k + 1], tv[3 * k + 2]));
+          D3 p, nn;
+          double d;
+          (void)sphere_triangle(w.s.dims[0], w.T2.t, P[0], P[1], P[2], p, d, nn);
+          nn = shp::neg(nn);  // the leaf stores minus the solver's normal
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            L.contact_pos[3 * slot + j] = p.v[j];
+            L.contact_normal[3 * slot + j] = nn.v[j];
+          }
+          L.contact_depth[slot] = d;
+        }
+      }
+    });
+  }
+  if (g.lane == 0) {
+    L.counts[q] = T.count;
+    if constexpr (kStats) {
+      L.stats[2 * q] = T.bv;
+      L.stats[2 * q + 1] = T.leaf;
+    }
+  }
 }
 
 // Lanes of a wavefront step together: a lane whose descent reached a leaf
@@ -490,68 +643,48 @@ __device__ __noinline__ bool leaf_test_gjk(const shp::Shape& s, const shp::Xf& T
 // own order of tests is the reference's, so counts, triangles and test
 // statistics are unchanged.
 //
-// kDeep: the pending right children live in device memory (deep_stack, one
-// column of L.max_depth entries per lane, lane-interleaved) instead of LDS,
-// for contexts holding a mesh deeper than kMsStack levels.
-//
-// kQueue (with kContact): hits that need EPA are queued (seeds, one
-// reservation per wavefront on nseed) instead of running EPA here.
-template <bool kContact, int kWaves, bool kDeep, bool kQueue = false>
-__global__ void __launch_bounds__(kBlk, kWaves) meshshape_collide(MeshShapeLaunch L,
-                                                                  const int32_t* order,
-                                                                  shp::EpaLane* lanes,
-                                                                  shp::EpaWave* waves,
-                                                                  int* deep_stack,
-                                                                  MsEpaSeed* seeds = nullptr,
-                                                                  unsigned long long* nseed =
-                                                                      nullptr) {
+// For what the lists in LDS do not hold: contexts with a mesh deeper than
+// kMsListDepth, and contact batches whose EPA queue would exceed its budget
+// (EPA then runs in the descending lane).  The pending right children live
+// in device memory (one column of L.max_depth entries per lane,
+// lane-interleaved).
+template <bool kContact>
+__global__ void __launch_bounds__(kBlk, 1) meshshape_deep(MeshShapeLaunch L, shp::EpaLane* lanes,
+                                                          shp::EpaWave* waves,
+                                                          int* deep_stack) {
   const size_t gid = static_cast<size_t>(blockIdx.x) * kBlk + threadIdx.x;
   const size_t stride = static_cast<size_t>(gridDim.x) * kBlk;
   // the horizon walk's stack in LDS, one column per thread
-  __shared__ int16_t xs_lds[(kContact && !kQueue) ? shp::kNfEpa : 1][kBlk];
+  __shared__ int16_t xs_lds[kContact ? shp::kNfEpa : 1][kBlk];
   shp::Epa E;
-  if constexpr (kContact && !kQueue) {
+  if constexpr (kContact) {
     E.M = lanes + gid;
     E.S = waves + gid / 64;
     E.lane = threadIdx.x & 63;
     E.xs = &xs_lds[0][threadIdx.x];
     E.xs_stride = kBlk;
   }
-  size_t qq = gid;  // position in the (sorted) order
-  size_t q = 0;     // the query at that position
+  size_t q = gid;
   shp::Shape s;
   shp::Xf T1, T2;
   double sa[9], sto[3], sext[3];
   const ObbNode64* nodes = nullptr;
   const double* tris = nullptr;
-  // pending right children in LDS, one column per lane (lane-interleaved:
-  // conflict-free whatever depth each lane is at); a deep stack holds at
-  // most L.max_depth - 1 entries
-  __shared__ int stk[kDeep ? 1 : kMsStack][kBlk];
-  const int col = threadIdx.x;
-  const int depth_max = kDeep ? L.max_depth : kMsStack;
   int sp = 0, b = 0, count = 0, pend = -1;
   long long nbv = 0, nleaf = 0;
   bool live = false;  // a query in progress
   auto push = [&](int v) {
-    if constexpr (kDeep)
-      deep_stack[static_cast<size_t>(sp) * stride + gid] = v;
-    else
-      stk[sp][col] = v;
+    deep_stack[static_cast<size_t>(sp) * stride + gid] = v;
     ++sp;
   };
   auto pop = [&]() -> int {
     --sp;
-    if constexpr (kDeep)
-      return deep_stack[static_cast<size_t>(sp) * stride + gid];
-    else
-      return stk[sp][col];
+    return deep_stack[static_cast<size_t>(sp) * stride + gid];
   };
   // take queries until one is usable (the others are answered at once)
   auto start = [&]() {
-    while (qq < static_cast<size_t>(L.num_queries)) {
-      q = order ? static_cast<size_t>(order[qq]) : qq;
-      if (load_query(L, static_cast<int>(q), s, depth_max)) {
+    while (q < static_cast<size_t>(L.num_queries)) {
+      if (load_query(L, static_cast<int>(q), s, L.max_depth)) {
         const MeshDev& M = L.meshes[L.query_meshes[q]];
         nodes = M.obb64;
         tris = M.tri_verts;
@@ -573,7 +706,7 @@ __global__ void __launch_bounds__(kBlk, kWaves) meshshape_collide(MeshShapeLaunc
         L.stats[2 * q + 1] = 0;
       }
       atomicOr(L.status, kStatusBadQuery);
-      qq += stride;
+      q += stride;
     }
     live = false;
   };
@@ -583,7 +716,7 @@ __global__ void __launch_bounds__(kBlk, kWaves) meshshape_collide(MeshShapeLaunc
       L.stats[2 * q] = nbv;
       L.stats[2 * q + 1] = nleaf;
     }
-    qq += stride;
+    q += stride;
     start();
   };
   auto next = [&]() {  // the next node of the descent, or the query's end
@@ -604,49 +737,19 @@ __global__ void __launch_bounds__(kBlk, kWaves) meshshape_collide(MeshShapeLaunc
       pend = -1;
       ++nleaf;
       shp::Contact c;
-      bool hit, need_epa = false;
-      shp::Gjk g;
-      const double* tv = tris + static_cast<size_t>(prim) * kTriVertsStride;
-      if constexpr (kQueue)
-        hit = leaf_test_gjk(s, T1, T2, tv, L.tol, c, g, need_epa);
-      else
-        hit = leaf_test<kContact>(s, T1, T2, tv, L.tol, E, c);
-      if constexpr (kQueue) {
-        // the seeds of this leaf round: one reservation for the wavefront
-        const unsigned long long em = __ballot(need_epa);
-        if (em != 0) {
-          const int leader = __ffsll(static_cast<long long>(em)) - 1;
-          unsigned long long b = 0;
-          if (static_cast<int>(threadIdx.x & 63) == leader)
-            b = atomicAdd(nseed, static_cast<unsigned long long>(__popcll(em)));
-          b = __shfl(b, leader);
-          if (need_epa) {
-            MsEpaSeed& sd =
-                seeds[b + __popcll(em & ((1ULL << (threadIdx.x & 63)) - 1ULL))];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              sd.w[j] = g.w[j];
-              sd.d[j] = g.d[j];
-            }
-            sd.q = static_cast<int32_t>(q);
-            sd.rank = g.rank;
-            sd.prim = prim;
-            sd.slot = static_cast<long long>(q * L.cap + count);
-          }
-        }
-      }
+      const bool hit =
+          leaf_test<kContact>(s, T1, T2, tris + static_cast<size_t>(prim) * kTriVertsStride, L.tol,
+                              E, c);
       if (hit) {
         const size_t k = q * L.cap + count;
         if (L.prims) L.prims[k] = prim;
         if constexpr (kContact) {
-          if (!need_epa) {
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-              L.contact_pos[3 * k + j] = c.pos.v[j];
-              L.contact_normal[3 * k + j] = c.normal.v[j];
-            }
-            L.contact_depth[k] = c.depth;
+          for (int j = 0; j < 3; ++j) {
+            L.contact_pos[3 * k + j] = c.pos.v[j];
+            L.contact_normal[3 * k + j] = c.normal.v[j];
           }
+          L.contact_depth[k] = c.depth;
         }
         if (++count >= L.cap) {
           finish();
@@ -733,13 +836,9 @@ __global__ void __launch_bounds__(kBlk, kWaves) meshshape_epa(MeshShapeLaunch L,
         const shp::Xf T1 = shp::xf_load(L.tf1 + 12 * static_cast<size_t>(q));
         T2 = shp::xf_load(L.tf2 + 12 * static_cast<size_t>(q));
         shp::make_mdiff(s, T2, tri, T1, m);
+        // GJK once more, for its final simplex ("inside", as the descent found)
         shp::Gjk g;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          g.w[j] = sd.w[j];
-          g.d[j] = sd.d[j];
-        }
-        g.rank = sd.rank;
+        (void)shp::gjk_evaluate(g, m, L.tol);
         slot = sd.slot;
         active = shp::epa_start(E, g, m, L.tol);
         finish = !active;
@@ -768,161 +867,110 @@ __global__ void __launch_bounds__(kBlk, kWaves) meshshape_epa(MeshShapeLaunch L,
 
 size_t mesh_shape_epa_lane_bytes() { return sizeof(shp::EpaLane) + sizeof(shp::EpaWave) / 64; }
 
-// the queued-EPA descent for a register budget of 1, 2 or 3 waves per SIMD
-void launch_queued(int waves, unsigned grid, hipStream_t s, const MeshShapeLaunch& L,
-                   const int32_t* order, MsEpaSeed* seeds, unsigned long long* nseed) {
-  switch (waves) {
-    case 1:
-      meshshape_collide<true, 1, false, true>
-          <<<grid, kBlk, 0, s>>>(L, order, nullptr, nullptr, nullptr, seeds, nseed);
-      break;
-    case 3:
-      meshshape_collide<true, 3, false, true>
-          <<<grid, kBlk, 0, s>>>(L, order, nullptr, nullptr, nullptr, seeds, nseed);
-      break;
-    default:
-      meshshape_collide<true, 2, false, true>
-          <<<grid, kBlk, 0, s>>>(L, order, nullptr, nullptr, nullptr, seeds, nseed);
-  }
-}
-
 __global__ void ms_zero_u64(unsigned long long* p) {
   if (threadIdx.x < 2) p[threadIdx.x] = 0;
 }
 
-template <bool kContact>
-void launch_variant(int waves, unsigned grid, hipStream_t s, const MeshShapeLaunch& L,
-                    const int32_t* order, shp::EpaLane* lanes, shp::EpaWave* wv,
-                    int* deep_stack) {
-  if (deep_stack) {
-    meshshape_collide<kContact, 1, true><<<grid, kBlk, 0, s>>>(L, order, lanes, wv, deep_stack);
-    return;
-  }
-  switch (waves) {
-    case 1:
-      meshshape_collide<kContact, 1, false><<<grid, kBlk, 0, s>>>(L, order, lanes, wv, nullptr);
-      break;
-    case 3:
-      meshshape_collide<kContact, 3, false><<<grid, kBlk, 0, s>>>(L, order, lanes, wv, nullptr);
-      break;
-    default:
-      meshshape_collide<kContact, 2, false><<<grid, kBlk, 0, s>>>(L, order, lanes, wv, nullptr);
-  }
+namespace {
+
+template <int kWaves>
+void launch_descent(const MeshShapeLaunch& L, const MsQuery* queries, MsEpaSeed* seeds,
+                    unsigned long long* nseed, hipStream_t s) {
+  auto kernel = L.contact ? (L.stats ? meshshape_ordered<true, true, kWaves>
+                                     : meshshape_ordered<false, true, kWaves>)
+                          : (L.stats ? meshshape_ordered<true, false, kWaves>
+                                     : meshshape_ordered<false, false, kWaves>);
+  const int leaf_min = L.leaf_share > 0 ? std::max(1, 64 * L.leaf_share / 100) : 64;
+  kernel<<<static_cast<unsigned>(L.num_queries), 64, 0, s>>>(L, queries, L.max_depth + 2, leaf_min,
+                                                             seeds, nseed);
 }
 
-// Batches at least this large are grouped by shape kind first.
-constexpr int kSortMin = 4096;
+// Stream-ordered scratch of one batch, freed (in stream order) at its end.
+struct StreamScratch {
+  hipStream_t s;
+  void* held[4] = {};
+  int n = 0;
+  explicit StreamScratch(hipStream_t stream) : s(stream) {}
+  ~StreamScratch() {
+    for (int i = 0; i < n; ++i) (void)hipFreeAsync(held[i], s);
+  }
+  template <typename T>
+  hipError_t get(T** p, size_t count) {
+    void* v = nullptr;
+    const hipError_t e = hipMallocAsync(&v, std::max<size_t>(count * sizeof(T), 16), s);
+    if (e == hipSuccess) {
+      held[n++] = v;
+      *p = static_cast<T*>(v);
+    }
+    return e;
+  }
+};
+
+#define MS_TRY(expr)                     \
+  do {                                   \
+    const hipError_t e_ = (expr);        \
+    if (e_ != hipSuccess) return e_;     \
+  } while (0)
+
+hipError_t launch_deep(MeshShapeLaunch L, int cus, hipStream_t s) {
+  // measured: leaf rounds at half the live lanes for booleans, three
+  // quarters with contact geometry
+  if (L.leaf_share <= 0) L.leaf_share = L.contact ? 75 : 50;
+  long long grid = (static_cast<long long>(L.num_queries) + kBlk - 1) / kBlk;
+  grid = std::min<long long>(grid, static_cast<long long>(cus) * kMsDeepBlocksPerCu);
+  const size_t lanes = static_cast<size_t>(grid) * kBlk;
+  StreamScratch mem(s);
+  int* stack = nullptr;
+  MS_TRY(mem.get(&stack, lanes * L.max_depth));
+  if (!L.contact) {
+    meshshape_deep<false><<<static_cast<unsigned>(grid), kBlk, 0, s>>>(L, nullptr, nullptr, stack);
+    return hipGetLastError();
+  }
+  shp::EpaLane* el = nullptr;
+  shp::EpaWave* ew = nullptr;
+  MS_TRY(mem.get(&el, lanes));
+  MS_TRY(mem.get(&ew, lanes / 64));
+  meshshape_deep<true><<<static_cast<unsigned>(grid), kBlk, 0, s>>>(L, el, ew, stack);
+  return hipGetLastError();
+}
+
+}  // namespace
 
 hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& in, int waves, hipStream_t s) {
   if (in.num_queries <= 0) return hipSuccess;
   MeshShapeLaunch L = in;
-  // measured: half the live lanes for booleans, three quarters with contact
-  // geometry (whose leaf rounds queue EPA's work for a pass of its own)
-  if (L.leaf_share <= 0) L.leaf_share = L.contact ? 75 : 50;
-  const long long blocks = (static_cast<long long>(L.num_queries) + kBlk - 1) / kBlk;
-  // the order of queries grouped by shape kind (stream-ordered memory)
-  int32_t* order = nullptr;
-  hipError_t e = hipSuccess;
-  if (L.num_queries >= kSortMin) {
-    e = hipMallocAsync(reinterpret_cast<void**>(&order),
-                       (static_cast<size_t>(L.num_queries) + 16) * sizeof(int32_t), s);
-    if (e != hipSuccess) return e;
-    int32_t* ctr = order + L.num_queries;
-    ms_zero<<<1, 64, 0, s>>>(ctr);
-    ms_count<<<static_cast<unsigned>(blocks), kBlk, 0, s>>>(L, ctr);
-    ms_place<<<static_cast<unsigned>(blocks), kBlk, 0, s>>>(L, ctr, order);
-  }
+  L.max_depth = std::min(L.max_depth, kMsDeepMax);  // deeper meshes are refused by load_query
   int dev = 0, cus = 0;
-  e = hipGetDevice(&dev);
-  if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (e != hipSuccess) {
-    if (order) (void)hipFreeAsync(order, s);
-    return e;
-  }
-  // a context with a mesh deeper than the LDS stack: a persistent grid whose
-  // lanes keep their stacks in device memory (queries on deeper meshes
-  // than kMsDeepMax are refused by load_query)
-  const bool deep = L.max_depth > kMsStack;
-  if (deep) L.max_depth = std::min(L.max_depth, kMsDeepMax);
-  long long grid = blocks;
-  if (deep) grid = std::min<long long>(grid, static_cast<long long>(cus) * kMsDeepBlocksPerCu);
-  if (L.contact) grid = std::min<long long>(grid, static_cast<long long>(cus) * kEpaBlocksPerCu);
-  int* deep_stack = nullptr;
-  if (deep) {
-    e = hipMallocAsync(reinterpret_cast<void**>(&deep_stack),
-                       static_cast<size_t>(grid) * kBlk * L.max_depth * sizeof(int), s);
-    if (e != hipSuccess) {
-      if (order) (void)hipFreeAsync(order, s);
-      return e;
-    }
-  }
-  if (!L.contact) {
-    launch_variant<false>(waves, static_cast<unsigned>(grid), s, L, order, nullptr, nullptr,
-                          deep_stack);
-    e = hipGetLastError();
-    if (deep_stack) (void)hipFreeAsync(deep_stack, s);
-    if (order) (void)hipFreeAsync(order, s);
-    return e;
-  }
-  // contacts with EPA queued: the descent on every query at once, then EPA
-  // on a persistent grid sized to its memory
+  MS_TRY(hipGetDevice(&dev));
+  MS_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const size_t nslots = static_cast<size_t>(L.num_queries) * static_cast<size_t>(L.cap);
-  if (!deep && nslots * sizeof(MsEpaSeed) <= kEpaQueueBudget) {
-    MsEpaSeed* seeds = nullptr;
-    unsigned long long* ctr = nullptr;  // [0] seeds queued, [1] seeds handed out
-    e = hipMallocAsync(reinterpret_cast<void**>(&seeds), nslots * sizeof(MsEpaSeed), s);
-    if (e == hipSuccess) {
-      e = hipMallocAsync(reinterpret_cast<void**>(&ctr), 2 * sizeof(unsigned long long), s);
-      if (e != hipSuccess) (void)hipFreeAsync(seeds, s);
-    }
-    if (e != hipSuccess) {
-      if (order) (void)hipFreeAsync(order, s);
-      return e;
-    }
+  if (L.max_depth > kMsListDepth || (L.contact && nslots > kEpaQueueBudget / sizeof(MsEpaSeed)))
+    return launch_deep(L, cus, s);
+  StreamScratch mem(s);
+  MsQuery* queries = nullptr;
+  MsEpaSeed* seeds = nullptr;
+  unsigned long long* ctr = nullptr;  // [0] seeds queued, [1] seeds handed out
+  MS_TRY(mem.get(&queries, static_cast<size_t>(L.num_queries)));
+  if (L.contact) {
+    MS_TRY(mem.get(&seeds, nslots));
+    MS_TRY(mem.get(&ctr, 2));
     ms_zero_u64<<<1, 64, 0, s>>>(ctr);
-    launch_queued(waves, static_cast<unsigned>(blocks), s, L, order, seeds, ctr);
-    e = hipGetLastError();
-    const long long egrid = static_cast<long long>(cus) * kEpaBlocksPerCu;
-    const size_t nl = static_cast<size_t>(egrid) * kBlk;
-    shp::EpaLane* lanes = nullptr;
-    shp::EpaWave* wv = nullptr;
-    if (e == hipSuccess) e = hipMallocAsync(reinterpret_cast<void**>(&lanes), nl * sizeof(shp::EpaLane), s);
-    if (e == hipSuccess) {
-      e = hipMallocAsync(reinterpret_cast<void**>(&wv), nl / 64 * sizeof(shp::EpaWave), s);
-      if (e != hipSuccess) (void)hipFreeAsync(lanes, s);
-    }
-    if (e == hipSuccess) {
-      meshshape_epa<2><<<static_cast<unsigned>(egrid), kBlk, 0, s>>>(L, seeds, ctr, ctr + 1,
-                                                                        lanes, wv);
-      e = hipGetLastError();
-      (void)hipFreeAsync(lanes, s);
-      (void)hipFreeAsync(wv, s);
-    }
-    (void)hipFreeAsync(seeds, s);
-    (void)hipFreeAsync(ctr, s);
-    if (order) (void)hipFreeAsync(order, s);
-    return e;
   }
-  const size_t nl = static_cast<size_t>(grid) * kBlk;
-  shp::EpaLane* lanes = nullptr;
-  shp::EpaWave* wv = nullptr;
-  e = hipMallocAsync(reinterpret_cast<void**>(&lanes), nl * sizeof(shp::EpaLane), s);
-  if (e == hipSuccess) {
-    e = hipMallocAsync(reinterpret_cast<void**>(&wv), nl / 64 * sizeof(shp::EpaWave), s);
-    if (e != hipSuccess) (void)hipFreeAsync(lanes, s);
-  }
-  if (e != hipSuccess) {
-    if (deep_stack) (void)hipFreeAsync(deep_stack, s);
-    if (order) (void)hipFreeAsync(order, s);
-    return e;
-  }
-  launch_variant<true>(waves, static_cast<unsigned>(grid), s, L, order, lanes, wv, deep_stack);
-  e = hipGetLastError();
-  (void)hipFreeAsync(lanes, s);
-  (void)hipFreeAsync(wv, s);
-  if (deep_stack) (void)hipFreeAsync(deep_stack, s);
-  if (order) (void)hipFreeAsync(order, s);
-  return e;
+  meshshape_setup<<<static_cast<unsigned>((L.num_queries + kBlk - 1) / kBlk), kBlk, 0, s>>>(
+      L, queries);
+  auto descent = waves == 1 ? launch_descent<1> : (waves == 3 ? launch_descent<3> : launch_descent<2>);
+  descent(L, queries, seeds, ctr, s);
+  MS_TRY(hipGetLastError());
+  if (!L.contact) return hipSuccess;
+  const long long egrid = static_cast<long long>(cus) * kEpaBlocksPerCu;
+  const size_t lanes = static_cast<size_t>(egrid) * kBlk;
+  StreamScratch emem(s);
+  shp::EpaLane* el = nullptr;
+  shp::EpaWave* ew = nullptr;
+  MS_TRY(emem.get(&el, lanes));
+  MS_TRY(emem.get(&ew, lanes / 64));
+  meshshape_epa<2><<<static_cast<unsigned>(egrid), kBlk, 0, s>>>(L, seeds, ctr, ctr + 1, el, ew);
+  return hipGetLastError();
 }
 
 }  // namespace fclx

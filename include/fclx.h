@@ -266,12 +266,11 @@ int fclx_collide_batch_noalloc(fclx_context* ctx, const fclx_collide_batch_args*
  * (mesh_shape_collision_traversal_node-inl.h:205-283).  Asynchronous; a
  * query naming a missing mesh or shape, an RSS mesh, a mesh deeper than 4096
  * levels or a convex with fewer than 4 vertices gets count 0 and makes
- * fclx_sync return FCLX_ERR_INVALID_ARGUMENT.  While the context holds a
- * mesh deeper than 64 levels, batches keep their descent stacks in
- * stream-ordered device memory (4 bytes per level per resident lane) instead
- * of LDS.  With enable_contact the call
- * takes stream-ordered device memory for EPA (about 12 KB per resident lane,
- * freed when the batch ends). */
+ * fclx_sync return FCLX_ERR_INVALID_ARGUMENT.  A call takes
+ * stream-ordered device memory, freed when the batch ends: 128 bytes per
+ * query, with enable_contact also for EPA (16 bytes per slot and about 12 KB
+ * per resident lane), and, while the context holds a mesh deeper than 440
+ * levels, for descent stacks (4 bytes per level per resident lane). */
 typedef struct {
   int32_t num_queries;
   const int32_t* query_meshes; /* device: mesh id per query */
@@ -397,10 +396,10 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *   "dist_waves_per_simd" 2, 3  register budget of the FAST distance kernel
  *   "meshshape_waves_per_simd" 1..3  register budget of the mesh-vs-primitive
  *                               kernel (default 2)
- *   "meshshape_leaf_share" 0..100  percent of a wavefront's live queries
- *                               waiting at leaves that starts their leaf
- *                               tests (default 0: 50 for booleans, 75
- *                               with contact geometry)
+ *   "meshshape_leaf_share" 0..100  percent of a wavefront's lanes with a leaf
+ *                               to test that starts their leaf tests
+ *                               (default 0: 100, or when nothing else is
+ *                               left to test)
  *   "dist_width"        1..64   most bounds of one query per distance step
  *                               (default 32)
  *   "dist_leaf_batch"   1..64   leaf pairs queued before their distances are
