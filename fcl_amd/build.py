@@ -18,7 +18,8 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libfclx.so")
 
-HIP_SOURCES = ["api.hip", "kernels_plain.hip", "kernels_ordered.hip", "kernels_front.hip", "kernels_refit.hip",
+HIP_SOURCES = ["api.hip", "kernels_plain.hip", "kernels_ordered.hip", "kernels_clearance.hip",
+               "kernels_front.hip", "kernels_refit.hip",
                "kernels_broadphase.hip",
                "kernels_shape.hip",
                "kernels_meshshape.hip",

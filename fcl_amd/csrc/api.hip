@@ -799,10 +799,12 @@ int fclx_distance_batch(fclx_context* ctx, const fclx_distance_batch_args* a, vo
   hipStream_t s = static_cast<hipStream_t>(stream);
   int depth, nmesh;
   bool merged;
+  size_t nodes;
   const MeshDev* table;
   {
     std::lock_guard<std::mutex> lock(ctx->mu);
     depth = max_depth(ctx);
+    nodes = max_nodes(ctx);
     nmesh = static_cast<int>(ctx->meshes.size());
     table = ctx->d_table;
     merged = any_merged(ctx);
@@ -831,9 +833,13 @@ int fclx_distance_batch(fclx_context* ctx, const fclx_distance_batch_args* a, vo
   // The FAST engine finds the reference's answer in any visit order only
   // when every bound is a lower bound of the pairs below it; merged BVs
   // need not be, and then only the reference's own order gives its answer.
-  hipError_t e = a->engine == FCLX_ENGINE_FAST && !merged
-                     ? launch_distance_wave(L, 2 * depth, tu, s)
-                     : launch_distance_plain(L, 2 * depth, s);
+  hipError_t e;
+  if (a->engine == FCLX_ENGINE_FAST && !merged)
+    e = launch_distance_wave(L, 2 * depth, tu, s);
+  else if (a->engine == FCLX_ENGINE_FAST && distance_ordered_takes(nodes))
+    e = launch_distance_ordered(L, 2 * depth, s);
+  else
+    e = launch_distance_plain(L, 2 * depth, s);
   if (e != hipSuccess) return hip_fail(ctx, e, "distance launch");
   return FCLX_OK;
 }
@@ -1501,7 +1507,10 @@ int fclx_distance(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_
   L.leaf_tests = ctx->s_stats + 1;
   L.status = ctx->d_status;
   const int depth = ctx->meshes[mesh1].bvh.depth + ctx->meshes[mesh2].bvh.depth;
-  HIP_TRY(ctx, launch_distance_plain(L, depth, s));
+  HIP_TRY(ctx, distance_ordered_takes(std::max(ctx->meshes[mesh1].bvh.nodes.size(),
+                                               ctx->meshes[mesh2].bvh.nodes.size()))
+                   ? launch_distance_ordered(L, depth, s)
+                   : launch_distance_plain(L, depth, s));
   double out[7];
   int32_t idv[2];
   long long st[2];

@@ -184,6 +184,10 @@ void shape_workspace_set_waves(ShapeWorkspace* w, int waves);
 size_t shape_epa_lane_bytes();
 hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_t s);
 hipError_t launch_distance_plain(const DistanceLaunch& L, int stack_need, hipStream_t s);
+// distance() in the reference's order, a wavefront per query
+// (kernels_clearance.hip); its entries hold node indices below 2^26
+bool distance_ordered_takes(size_t max_nodes);
+hipError_t launch_distance_ordered(const DistanceLaunch& L, int stack_need, hipStream_t s);
 // FAST engine: wavefront-wide search with the reference's visit order kept
 // as path keys (engine_dist.hip); BVTTs deeper than 62 levels go to the
 // plain kernel
