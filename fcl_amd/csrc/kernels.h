@@ -32,7 +32,8 @@ struct CollideLaunch {
   int32_t* counts;             // per query
   int32_t* pairs;              // 3 per record: query, b1, b2
   long long pair_capacity;
-  long long* num_pairs;        // running record count (may exceed capacity)
+  long long* num_pairs;        // running record count (may exceed capacity); NULL
+                               // for the ordered kernel's single queries
   long long* bv_tests;         // optional, per query
   long long* leaf_tests;       // optional, per query
   int32_t* status;             // device status word (kStatus* bits)

@@ -282,8 +282,8 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
     }
     ord_settle<G, kCap, kStats>(g, S, T, r, acc, n, L.cap, [&](bool mine, int take, int before,
                                                                int total) {
-      unsigned long long b = 0;
-      if (g.lane == 0 && total > 0)
+      unsigned long long b = static_cast<unsigned>(T.count);  // a single query's own records
+      if (L.num_pairs && g.lane == 0 && total > 0)
         b = atomicAdd(reinterpret_cast<unsigned long long*>(L.num_pairs),
                       static_cast<unsigned long long>(total));
       b = (static_cast<unsigned long long>(g.at(static_cast<unsigned>(b >> 32), 0)) << 32) |
