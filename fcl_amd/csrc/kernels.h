@@ -174,7 +174,7 @@ struct RefitLaunch {
 // level_offsets_host[l] .. [l+1] (host array of levels + 1) bounding each.
 hipError_t launch_refit(const RefitLaunch& L, bool bottomup, const int32_t* level_nodes,
                         const int32_t* level_offsets_host, int levels, hipStream_t s);
-// Sort buffers, the EPA queue and per-lane EPA memory of the shape path; one
+// Sort buffers and the EPA queue of the shape path; one
 // per context, used by one batch at a time (the caller serialises calls;
 // batches on different streams are ordered through an event).
 struct ShapeWorkspace;
@@ -182,7 +182,6 @@ ShapeWorkspace* shape_workspace_create(int device);
 void shape_workspace_destroy(ShapeWorkspace* w);
 void shape_workspace_set_epa_blocks_per_cu(ShapeWorkspace* w, int blocks);
 void shape_workspace_set_waves(ShapeWorkspace* w, int waves);
-size_t shape_epa_lane_bytes();
 hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_t s);
 hipError_t launch_distance_plain(const DistanceLaunch& L, int stack_need, hipStream_t s);
 // distance() in the reference's order, a wavefront per query

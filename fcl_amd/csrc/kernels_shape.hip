@@ -14,18 +14,17 @@
 //      them it collides, and EPA -- whose status is never Failed after GJK's
 //      Inside -- would only have supplied the contact);
 //   3. EPA over the queue (GJK's final simplex per pair): a persistent grid
-//      in which every lane runs its own pair one EPA loop pass at a time and
-//      takes the next pair of its wavefront's share when done, so lanes do
-//      not wait for the slowest pair of their wavefront; a lane keeps EPA's
-//      faces and vertices in a contiguous block of device memory of its own.
+//      of lane groups, each with one pair's polytope in LDS, taking the next
+//      pair when done; then the pairs whose polytopes outgrew those stores,
+//      from the start, in stores of the reference's full size.
 // Same-address atomics are kept few: one per block per counter in the
-// sorting and GJK kernels (the GJK kernel's on per-XCD counters), one per 64
-// pairs in EPA.
+// sorting and GJK kernels (the GJK kernel's on per-XCD counters), one per
+// wavefront's idle groups in EPA.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
-#include "device/shape64.h"
+#include "device/epa_group.h"
 #include "kernels.h"
 
 namespace fclx {
@@ -48,6 +47,8 @@ enum : int {
   kCtrValid,                     // well-formed pairs (positions [0, valid))
   kCtrQueue,                     // pairs queued for EPA, per XCD sub-queue (8)
   kCtrGrab = kCtrQueue + 8,      // EPA queue entries handed to wavefronts
+  kCtrSpill,                     // pairs the small EPA store could not hold
+  kCtrSpillGrab,                 // of those, handed to wavefronts
   kNumCtr
 };
 
@@ -275,101 +276,75 @@ __global__ void __launch_bounds__(kBlk, kWaves) shape_gjk(ShapeLaunch L, const i
   }
 }
 
-// Idle lanes of a wavefront take new pairs once this many are idle (or all).
-constexpr int kRefill = 16;
-
-// EPA over the queued pairs (the sub-queues, concatenated).  A wavefront
-// takes 64 entries at a time with one atomic; every lane runs its own pair
-// one loop pass per trip and takes the wavefront's next entry when done, so
-// lanes do not wait for the slowest pair of their wavefront.
-template <int kWaves>
-__global__ void __launch_bounds__(kBlk, kWaves) shape_epa(ShapeLaunch L,
-                                                          const shp::EpaSeed* seeds,
-                                                          int32_t* ctr, int sub_cap,
-                                                          shp::EpaLane* lanes,
-                                                          shp::EpaWave* waves) {
-  const int lane = threadIdx.x & 63;
-  const size_t gid = static_cast<size_t>(blockIdx.x) * kBlk + threadIdx.x;
-  int sub_end[8];  // running totals of the sub-queue sizes
+// EPA over the queued pairs, a group of lanes each (device/epa_group.h): first
+// the queue (the sub-queues, concatenated) with small stores, then the pairs
+// those could not hold with stores of the reference's size.
+//
+// Bound: the horizon walk, a serial chain of LDS reads (two thirds of a pass);
+// then latency at 8 wavefronts per CU, which the LDS allows.  With a lane per
+// pair the polytopes (11.6 KB each, 131,072 of them) were in device memory,
+// and the walk's scattered reads moved whole lines from HBM.  1,000,000 pairs
+// (200,000 of them in here): 7.5 ms -> 4.6 + 1.8; the whole call 8.7 -> 7.7 ms
+// for 1,000,000 pairs, 5.1 -> 1.8 for 100,000, 2.7 -> 1.1 for 1,000.
+template <typename Store, int G>
+__global__ void __launch_bounds__(shp::kEpaBlock, 2) shape_epa(ShapeLaunch L,
+                                                               const shp::EpaSeed* seeds,
+                                                               int32_t* ctr, int sub_cap,
+                                                               const int32_t* todo,
+                                                               int32_t* spill) {
+  __shared__ Store stores[shp::kEpaBlock / G];
+  struct Job {
+    const ShapeLaunch& L;
+    const shp::EpaSeed* seeds;
+    const int32_t* todo;
+    int32_t* spilled;
+    int32_t* nspill;
+    int sub_cap, sub_end[8];  // running totals of the sub-queue sizes
+    int entry, q, gjk_passes;
+    __device__ __forceinline__ void load(long long v, shp::MDiff& m, shp::Gjk& g) {
+      entry = todo ? todo[v] : static_cast<int>(v);
+      int x = 0, before = 0;
+#pragma unroll
+      for (int k = 0; k < 7; ++k)
+        if (entry >= sub_end[k]) {
+          x = k + 1;
+          before = sub_end[k];
+        }
+      const shp::EpaSeed& sd = seeds[static_cast<size_t>(x) * sub_cap + (entry - before)];
+      q = sd.q;
+      gjk_passes = sd.gjk_passes;
+      shp::Shape s1, s2;
+      load_shape(L, L.pair_shapes[2 * q], s1);
+      load_shape(L, L.pair_shapes[2 * q + 1], s2);
+      shp::make_mdiff(s1, pose(), s2, shp::xf_load(L.tf2 + 12 * static_cast<size_t>(q)), m);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        g.w[k] = sd.w[k];
+        g.d[k] = sd.d[k];
+      }
+      g.rank = sd.rank;
+    }
+    __device__ __forceinline__ shp::Xf pose() const {
+      return shp::xf_load(L.tf1 + 12 * static_cast<size_t>(q));
+    }
+    __device__ __forceinline__ void done(const shp::Contact& c, int epa_passes) {
+      write_contacts(L, q, &c, 1);
+      if (L.passes) {
+        L.passes[2 * q] = gjk_passes;
+        L.passes[2 * q + 1] = epa_passes;
+      }
+    }
+    __device__ __forceinline__ void spill() { spilled[atomicAdd(nspill, 1)] = entry; }
+  };
+  Job job{L, seeds, todo, spill, &ctr[kCtrSpill], sub_cap, {}, 0, 0, 0};
   int total = 0;
 #pragma unroll
   for (int x = 0; x < 8; ++x) {
     total += ctr[kCtrQueue + x];
-    sub_end[x] = total;
+    job.sub_end[x] = total;
   }
-  const int wid = static_cast<int>(gid / 64);
-  int cursor = 0, stop = 0;  // the wavefront's entries not yet started
-  bool exhausted = false;
-  // the horizon walk's stack in LDS, one column per thread (a frame is
-  // popped right after the walk returns from a child, at LDS latency)
-  __shared__ int16_t xs_lds[shp::kNfEpa][kBlk];
-  shp::Epa E;
-  E.M = lanes + gid;
-  E.S = waves + wid;
-  E.lane = lane;
-  E.xs = &xs_lds[0][threadIdx.x];
-  E.xs_stride = kBlk;
-  shp::MDiff m;
-  int q = -1, gjk_passes = 0;
-  bool active = false;
-  while (true) {
-    bool finish = false, started = false;
-    const unsigned long long idle = __ballot(!active);
-    const int nidle = __popcll(idle);
-    if (cursor >= stop && !exhausted && (nidle == 64 || nidle >= kRefill)) {
-      int base = 0;
-      if (lane == 0) base = atomicAdd(&ctr[kCtrGrab], 64);
-      base = __shfl(base, 0);
-      cursor = base < total ? base : total;
-      stop = base + 64 < total ? base + 64 : total;
-      exhausted = base + 64 >= total;
-    }
-    if (cursor < stop && (nidle == 64 || nidle >= kRefill)) {
-      const int v = cursor + __popcll(idle & ((1ull << lane) - 1));
-      cursor = cursor + nidle < stop ? cursor + nidle : stop;
-      if (!active && v < stop) {
-        int x = 0, before = 0;
-#pragma unroll
-        for (int k = 0; k < 7; ++k)
-          if (v >= sub_end[k]) {
-            x = k + 1;
-            before = sub_end[k];
-          }
-        const shp::EpaSeed& sd = seeds[static_cast<size_t>(x) * sub_cap + (v - before)];
-        q = sd.q;
-        gjk_passes = sd.gjk_passes;
-        shp::Shape s1, s2;
-        load_shape(L, L.pair_shapes[2 * q], s1);
-        load_shape(L, L.pair_shapes[2 * q + 1], s2);
-        shp::make_mdiff(s1, shp::xf_load(L.tf1 + 12 * static_cast<size_t>(q)), s2,
-                        shp::xf_load(L.tf2 + 12 * static_cast<size_t>(q)), m);
-        shp::Gjk g;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          g.w[k] = sd.w[k];
-          g.d[k] = sd.d[k];
-        }
-        g.rank = sd.rank;
-        active = shp::epa_start(E, g, m, L.tol);
-        finish = !active;
-        started = true;
-      }
-    }
-    if (active && !started) {
-      active = shp::epa_step(E, m, L.tol);
-      finish = !active;
-    }
-    if (finish) {
-      const shp::Contact c =
-          shp::epa_finish(E, m, shp::xf_load(L.tf1 + 12 * static_cast<size_t>(q)));
-      write_contacts(L, q, &c, 1);
-      if (L.passes) {
-        L.passes[2 * q] = gjk_passes;
-        L.passes[2 * q + 1] = E.fallback ? 0 : E.it;
-      }
-    }
-    if (exhausted && cursor >= stop && !__ballot(active)) break;
-  }
+  if (todo) total = ctr[kCtrSpill];
+  shp::epa_groups<G>(job, stores, total, &ctr[todo ? kCtrSpillGrab : kCtrGrab], L.tol);
 }
 
 }  // namespace
@@ -382,11 +357,8 @@ struct ShapeWorkspace {
   shp::EpaSeed* seeds = nullptr;  // EPA queue (allocated with enable_contact)
   long long seed_cap = 0;
   int32_t* ctr = nullptr;
-  shp::EpaLane* epa = nullptr;
-  shp::EpaWave* epa_waves = nullptr;
-  int epa_blocks = 0;
-  int epa_blocks_per_cu = 0;  // 0: as many as are resident
-  int waves = 2;              // register budget of the GJK and EPA kernels (waves per SIMD)
+  int epa_blocks_per_cu = 0;  // 0: as many as fit
+  int waves = 2;              // register budget of the GJK kernel (waves per SIMD)
   hipEvent_t done = nullptr;
   bool pending = false;       // done marks the last batch's end
 };
@@ -413,8 +385,6 @@ void shape_workspace_destroy(ShapeWorkspace* w) {
   if (w->pending) (void)hipEventSynchronize(w->done);
   release_buffers(w);
   (void)hipFree(w->ctr);
-  (void)hipFree(w->epa);
-  (void)hipFree(w->epa_waves);
   if (w->done) (void)hipEventDestroy(w->done);
   delete w;
 }
@@ -427,42 +397,14 @@ void shape_workspace_set_waves(ShapeWorkspace* w, int waves) { w->waves = waves;
 
 namespace {
 
-// GJK and EPA kernels for a register budget of 2, 3 or 4 waves per SIMD
-struct ShapeKernels {
-  const void* epa;
-  void (*launch_gjk)(int, hipStream_t, const ShapeLaunch&, const int32_t*, int32_t*,
-                     shp::EpaSeed*, int);
-  void (*launch_epa)(int, hipStream_t, const ShapeLaunch&, const shp::EpaSeed*, int32_t*,
-                     int, shp::EpaLane*, shp::EpaWave*);
-};
+using GjkKernel = void (*)(ShapeLaunch, const int32_t*, int32_t*, shp::EpaSeed*, int);
 
-template <int W>
-ShapeKernels kernels_for() {
-  return {reinterpret_cast<const void*>(&shape_epa<W>),
-          [](int grid, hipStream_t s, const ShapeLaunch& L, const int32_t* perm, int32_t* ctr,
-             shp::EpaSeed* seeds, int sub_cap) {
-            shape_gjk<W><<<grid, kBlk, 0, s>>>(L, perm, ctr, seeds, sub_cap);
-          },
-          [](int grid, hipStream_t s, const ShapeLaunch& L, const shp::EpaSeed* seeds,
-             int32_t* ctr, int sub_cap, shp::EpaLane* lanes, shp::EpaWave* waves) {
-            shape_epa<W><<<grid, kBlk, 0, s>>>(L, seeds, ctr, sub_cap, lanes, waves);
-          }};
-}
-
-ShapeKernels select_kernels(int waves) {
-  switch (waves) {
-    case 3:
-      return kernels_for<3>();
-    case 4:
-      return kernels_for<4>();
-    default:
-      return kernels_for<2>();
-  }
+// the GJK kernel for a register budget of 2, 3 or 4 waves per SIMD
+GjkKernel gjk_kernel(int waves) {
+  return waves == 3 ? shape_gjk<3> : (waves == 4 ? shape_gjk<4> : shape_gjk<2>);
 }
 
 }  // namespace
-
-size_t shape_epa_lane_bytes() { return sizeof(shp::EpaLane) + sizeof(shp::EpaWave) / 64; }
 
 hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_t s) {
   if (L.num_pairs <= 0) return hipSuccess;
@@ -470,23 +412,19 @@ hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_
   if (!w->done && (e = hipEventCreateWithFlags(&w->done, hipEventDisableTiming)) != hipSuccess)
     return e;
   if (!w->ctr && (e = hipMalloc(&w->ctr, sizeof(int32_t) * kNumCtr)) != hipSuccess) return e;
-  // the EPA grid: resident blocks on every CU (or the set cap per CU)
-  int cus = 0, resident = 0;
+  // the EPA grid: the blocks that LDS has room for (or the set cap per CU)
+  int cus = 0;
   if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, w->device)) !=
       hipSuccess)
     return e;
-  const ShapeKernels K = select_kernels(w->waves);
-  if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, K.epa, kBlk, 0)) !=
-      hipSuccess)
-    return e;
-  resident = std::max(1, resident);
-  if (w->epa_blocks_per_cu > 0) resident = std::min(resident, w->epa_blocks_per_cu);
-  const int epa_blocks = cus * resident;
+  const int epa_blocks = cus * (w->epa_blocks_per_cu > 0
+                                    ? std::min(w->epa_blocks_per_cu, shp::kEpaBlocksPerCu)
+                                    : shp::kEpaBlocksPerCu);
   const int n = L.num_pairs;
   const int grid = (n + kBlk - 1) / kBlk;
   const int sub_cap = (grid + 7) / 8 * kBlk;
   const bool grow = n > w->cap || (L.contact && 8LL * sub_cap > w->seed_cap);
-  if ((grow || epa_blocks != w->epa_blocks) && w->pending) {
+  if (grow && w->pending) {
     if ((e = hipEventSynchronize(w->done)) != hipSuccess) return e;
     w->pending = false;
   }
@@ -503,18 +441,6 @@ hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_
     w->cap = cap;
     w->seed_cap = seed_cap;
   }
-  if (epa_blocks != w->epa_blocks) {
-    (void)hipFree(w->epa);
-    (void)hipFree(w->epa_waves);
-    w->epa = nullptr;
-    w->epa_waves = nullptr;
-    w->epa_blocks = 0;
-    const size_t lanes = static_cast<size_t>(epa_blocks) * kBlk;
-    if ((e = hipMalloc(&w->epa, sizeof(shp::EpaLane) * lanes)) != hipSuccess ||
-        (e = hipMalloc(&w->epa_waves, sizeof(shp::EpaWave) * (lanes / 64))) != hipSuccess)
-      return e;
-    w->epa_blocks = epa_blocks;
-  }
   // a batch on another stream may still be using the buffers
   if (w->pending && (e = hipStreamWaitEvent(s, w->done, 0)) != hipSuccess) return e;
 
@@ -524,9 +450,14 @@ hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_
   shape_scan<<<1, 64, 0, s>>>(w->ctr);
   shape_scatter<<<sort_grid, kBlk, 0, s>>>(n, w->keys, w->ctr, w->perm);
   shape_closed<<<grid, kBlk, 0, s>>>(L, w->perm, w->ctr);
-  K.launch_gjk(grid, s, L, w->perm, w->ctr, w->seeds, sub_cap);
-  if (L.contact)
-    K.launch_epa(w->epa_blocks, s, L, w->seeds, w->ctr, sub_cap, w->epa, w->epa_waves);
+  gjk_kernel(w->waves)<<<grid, kBlk, 0, s>>>(L, w->perm, w->ctr, w->seeds, sub_cap);
+  if (L.contact) {
+    // (the sorted positions are done with: their array takes the spilled entries)
+    shape_epa<shp::EpaSmall, shp::kEpaSmallLanes><<<epa_blocks, shp::kEpaBlock, 0, s>>>(
+        L, w->seeds, w->ctr, sub_cap, nullptr, w->perm);
+    shape_epa<shp::EpaLarge, shp::kEpaLargeLanes><<<epa_blocks, shp::kEpaBlock, 0, s>>>(
+        L, w->seeds, w->ctr, sub_cap, w->perm, nullptr);
+  }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if ((e = hipEventRecord(w->done, s)) != hipSuccess) return e;
   w->pending = true;

@@ -419,11 +419,10 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               children of a node stay; same outputs
  *                               (default 0: FP64 bounds throughout, faster
  *                               on MI355X)
- *   "epa_blocks_per_cu" 0..32   resident blocks per CU of the shape path's EPA
- *                               kernel (0: as many as fit); each lane holds
- *                               a 13 KiB EPA block in device memory
- *   "shape_waves_per_simd" 2..4 register budget of the shape path's GJK and
- *                               EPA kernels (default 2)
+ *   "epa_blocks_per_cu" 0..32   most blocks per CU of the shape path's EPA
+ *                               kernels (0: the two that LDS has room for)
+ *   "shape_waves_per_simd" 2..4 register budget of the shape path's GJK
+ *                               kernel (default 2)
  * Results do not depend on them; smaller buffers mean more rounds. */
 int fclx_set_engine_param(fclx_context* ctx, const char* name, double value);
 /* The current value of a tunable above (for tuners); no reference
