@@ -192,11 +192,11 @@ hipError_t launch_distance_ordered(const DistanceLaunch& L, int stack_need, hipS
 // as path keys (engine_dist.hip); BVTTs deeper than 62 levels go to the
 // plain kernel
 struct DistanceTuning {
-  int queries_per_wave = 4;  // 2, 4, 8: at most
+  int queries_per_wave = 4;  // 2, 4, 8
   int waves_per_simd = 2;    // 2, 3
-  int width = 32;            // most tasks of one query per step
-  int leaf_batch = 32;       // leaf pairs queued before their distances are taken
-  int fp32_cull = 1;         // 1: FP32 intervals first, FP64 where they decide nothing
+  int width = 32;            // most bounds of one query per step
+  int leaf_batch = 16;       // leaf pairs queued before their distances are taken
+  int fp32_cull = 0;         // 1: FP32 lower bounds first, FP64 where both children stay
 };
 hipError_t launch_distance_wave(const DistanceLaunch& L, int stack_need, const DistanceTuning& tu,
                                 hipStream_t s);

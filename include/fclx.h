@@ -391,8 +391,8 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               default 16)
  *   "bool_refill"       1..32   free query slots that make a BOOL-engine
  *                               wavefront take new queries (default 4)
- *   "dist_queries_per_wave" 2, 4, 8  most queries a FAST distance wavefront
- *                               keeps in flight (default 4)
+ *   "dist_queries_per_wave" 2, 4, 8  queries a FAST distance wavefront keeps
+ *                               in flight (default 4)
  *   "dist_waves_per_simd" 2, 3  register budget of the FAST distance kernel
  *   "meshshape_waves_per_simd" 1..3  register budget of the mesh-vs-primitive
  *                               kernel (default 2)
@@ -400,10 +400,10 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               to test that starts their leaf tests
  *                               (default 0: 100, or when nothing else is
  *                               left to test)
- *   "dist_width"        1..64   most node pairs of one query expanded per
- *                               distance step (32 at most are; default 32)
+ *   "dist_width"        1..64   most bounds of one query per distance step
+ *                               (default 32)
  *   "dist_leaf_batch"   1..64   leaf pairs queued before their distances are
- *                               taken (default 32)
+ *                               taken (default 16)
  *   "fast_persistent"   0, 1    1: FAST collide batches with caps above 64 run
  *                               as one persistent launch (the BOOL kernel's
  *                               exhaustive form: per-query slots fed from
@@ -413,11 +413,12 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *   "fast_graph"        0, 1    1: that launch sequence is captured once in a
  *                               HIP graph and replayed while its arguments
  *                               stay the same (default 1)
- *   "dist_fp32_cull"    0, 1    1: FAST distance takes certified FP32
- *                               intervals of the RSS distances first (64-B
- *                               float nodes) and FP64 bounds only where those
- *                               decide nothing (default); 0: FP64 bounds
- *                               throughout; same outputs
+ *   "dist_fp32_cull"    0, 1    1: FAST distance takes certified FP32 lower
+ *                               bounds of the RSS distances first (64-B
+ *                               float nodes) and FP64 bounds only where both
+ *                               children of a node stay; same outputs
+ *                               (default 0: FP64 bounds throughout, faster
+ *                               on MI355X)
  *   "epa_blocks_per_cu" 0..32   most blocks per CU of the shape path's EPA
  *                               kernels (0: the two that LDS has room for)
  *   "shape_waves_per_simd" 2..4 register budget of the shape path's GJK
