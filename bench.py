@@ -552,7 +552,7 @@ def bench_meshshape(args):
     ops = w_bv * OPS_BV + w_leaf * OPS_GJK_PASS
     alg_bytes = w_bv * BYTES_BV64 + w_leaf * BYTES_LEAF_TRI
     roofline = {
-        "kernel": "meshshape_collide<false> (one query per lane, FP64)",
+        "kernel": "meshshape_ordered (a wavefront per query)",
         "bound": "valu",
         "achieved": ops / t_k / 1e12,
         "peak": PEAK_FP64 / 1e12,

@@ -55,7 +55,7 @@ extern "C" {
  * a query come out in no particular order).  A query that reaches the cap
  * gets the reference's depth-first prefix, in order: its records are ordered
  * by depth-first path keys and cut, or, when per-query statistics are
- * requested, the query is re-run by PLAIN.  Batches over a context holding
+ * requested, the query is re-run in that order.  Batches over a context holding
  * a mesh of 2^20 or more triangles, and batches of 2^22 or more queries, run
  * PLAIN for caps above 64 (the FAST engine's task encoding has 21 bits per
  * node index and 22 per query). */
@@ -100,7 +100,7 @@ typedef struct {
   /* CollisionRequest::enable_contact (mesh_collision_traversal_node-inl.h:
    * 578-598): each record is one contact (a triangle pair gives 0-2), counts
    * and num_max_contacts count contacts, and the geometry below is written
-   * per record in the world frame.  Runs the reference-order kernel whatever
+   * per record in the world frame.  Runs in the reference's order whatever
    * the engine.  The three arrays are required when pairs is set. */
   int32_t enable_contact;
   int32_t reserved;
@@ -215,8 +215,8 @@ int fclx_mesh_export_nodes(fclx_context* ctx, int32_t mesh_id, double* bv_data,
  * both children, so after a bottom-up refit a BV's RSS distance is not
  * always a lower bound of the triangle pairs below it, and distance()
  * depends on the visit order: while any mesh of the context holds merged
- * BVs, FCLX_ENGINE_FAST distance batches run the reference-order PLAIN
- * kernel (a top-down refit clears this).  Collide batches are unaffected:
+ * BVs, FCLX_ENGINE_FAST distance batches run in the reference's order (a
+ * top-down refit clears this).  Collide batches are unaffected:
  * their results do not depend on the visit order. */
 int fclx_mesh_refit(fclx_context* ctx, int32_t mesh_id, const double* vertices,
                     int32_t bottomup, void* stream);
