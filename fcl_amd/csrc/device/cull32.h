@@ -20,6 +20,11 @@
 //   d'_k >  M  for some k  =>  the FP64 test finds that axis separating;
 //   d'_k <= -M for every k =>  the FP64 test finds no separating axis;
 //   otherwise the caller runs the FP64 test.
+// The relative bounds hold while no term leaves FP32's normal range.  Below
+// it every conversion and operation is off by at most 2^-126 more (some 200 of
+// them, with factors <= 1.1), which the absolute kCullTiny in X.ms covers.
+// Above it, M < kCullHuge = 2^100 means S_T < 2^118 and extents < 2^120, so
+// that nothing has overflowed; any larger (or unordered) M is left to FP64.
 // Either sure outcome is the FP64 outcome, so culling visits exactly the
 // reference's set of BVTT nodes.
 #pragma once
@@ -32,11 +37,14 @@ namespace fclx {
 constexpr float kCullU = 5.9604644775390625e-08f;  // 2^-24
 constexpr float kCullKS = 68.0f;
 constexpr float kCullKR = 22.0f;
+constexpr float kCullTiny = 7.8886090522101181e-31f;  // 2^-100
+constexpr float kCullHuge = 1.2676506002282294e+30f;  // 2^100
 
 enum CullResult : int { kCullDisjoint = 0, kCullOverlap = 1, kCullUnsure = 2 };
 
-// Query transform in float plus its translation-margin term KS*u*S_T
-// (S_T includes the largest |c|_1 of either mesh's nodes).
+// Query transform in float plus its translation-margin term KS*u*S_T +
+// kCullTiny (S_T includes the largest |c|_1 of either mesh's nodes); INFINITY
+// leaves every test to FP64.
 struct alignas(64) QueryXf32 {
   float R[9];
   float T[3];
@@ -118,7 +126,7 @@ __device__ __forceinline__ int obb_cull32(const QueryXf32& X, const ObbNode32& n
       acc(fabsf(s) - r);
     }
   }
-  if (nan || !(M == M)) return kCullUnsure;
+  if (nan || !(M < kCullHuge)) return kCullUnsure;
   if (dmax > M) return kCullDisjoint;
   if (dmax <= -M) return kCullOverlap;
   return kCullUnsure;

@@ -57,7 +57,8 @@ __device__ __forceinline__ void make_xf32(const double* R, const double* T, doub
   for (int i = 0; i < 3; ++i) X.T[i] = static_cast<float>(T[i]);
   const double st = cmax1 + (fabs(T[0]) + fabs(T[1]) + fabs(T[2])) + cmax2;
   // margin rounded up: the float conversion may round down by <= 2^-24
-  X.ms = static_cast<float>(static_cast<double>(kCullKS) * static_cast<double>(kCullU) * st *
+  X.ms = static_cast<float>((static_cast<double>(kCullKS) * static_cast<double>(kCullU) * st +
+                             static_cast<double>(kCullTiny)) *
                             (1.0 + 1.0 / 1048576.0));
 }
 

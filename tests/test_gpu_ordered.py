@@ -85,3 +85,33 @@ def test_a_full_list_of_hits(ctx):
     pairs, stats = ctx.collide(m[0], tf1[0], m[1], tf2[0], cap=100000)
     assert len(pairs) > 200 and np.array_equal(pairs, a[2][0])
     assert stats.tolist() == [a[3][0], a[4][0]]
+
+
+@pytest.mark.parametrize("scale", [1e-45, 1e-41, 1e-30, 1e30, 1e38])
+def test_sizes_at_the_ends_of_floats(scale):
+    """Coordinates that floats hold badly or not at all: the single calls and
+    every batch answer as FP64 does."""
+    n = 80
+    print("case: ordered groups, sizes of %g" % scale, flush=True)
+    local = F.Context(0)
+    A, B = F.icosphere(5, 0.15, 3), F.icosphere(5, 0.15, 4)
+    m = [local.mesh(A[0] * scale, A[1]), local.mesh(B[0] * scale, B[1])]
+    tf1, tf2 = F.poses(n, 0, 1.7, 0, 0xE4D)
+    tf1[:, 9:] *= scale
+    tf2[:, 9:] *= scale
+    qm = np.tile(np.array(m, np.int32), (n, 1))
+    for cap in (1, 5):
+        _same(local, qm, tf1, tf2, cap, True)
+    # every contact: the batch gives each query's in any order
+    want, got = [collide_gpu(local, qm, tf1, tf2, 100000, engine=e, capacity=1 << 20)
+                 for e in (F.ENGINE_PLAIN, F.ENGINE_FAST)]
+    assert want[0] == got[0] == 0 and want[5] == got[5]
+    assert all(np.array_equal(want[k], got[k]) for k in (1, 3, 4))
+    for q, pairs in want[2].items():
+        assert np.array_equal(*[p[np.lexsort(p.T)] for p in (pairs, got[2][q])])
+    assert 0 < (want[1] > 0).mean() < 1
+    for q in range(0, n, 3):
+        pairs, stats = local.collide(m[0], tf1[q], m[1], tf2[q], cap=100000)
+        assert np.array_equal(pairs, want[2].get(q, np.zeros((0, 2))))
+        assert stats.tolist() == [want[3][q], want[4][q]]
+    local.close()
