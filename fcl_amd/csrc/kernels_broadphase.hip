@@ -146,20 +146,47 @@ __global__ void bp_clear(int n, uint32_t* count) {
   if (i < n) count[i] = 0;
 }
 
+// The box of the largest ordered (not NaN) lower x, the last of them in the
+// sweep's order; at < 0: there is none.  Found by the whole wavefront.
+struct LastBox {
+  double lo;
+  int at;
+};
+__device__ __noinline__ LastBox last_ordered(int n, const double* aabbs) {
+  unsigned long long bits = 0;
+  LastBox r{0.0, -1};
+  for (int k = static_cast<int>(__lane_id()); k < n; k += kWave) {
+    const double lo = aabbs[6 * static_cast<size_t>(k)];
+    const unsigned long long u = order_bits(lo);
+    if (lo == lo && (r.at < 0 || u >= bits)) {
+      bits = u;
+      r = LastBox{lo, k};
+    }
+  }
+  for (int d = 1; d < kWave; d <<= 1) {
+    const unsigned long long u = __shfl_xor(bits, d);
+    const LastBox o{__shfl_xor(r.lo, d), __shfl_xor(r.at, d)};
+    if (o.at >= 0 && (r.at < 0 || u > bits || (u == bits && o.at > r.at))) {
+      bits = u;
+      r = o;
+    }
+  }
+  return r;
+}
+
 // The sweep meets a box whose lower x is NaN (sorted last) only from objects
-// whose walk no ordered lower x ends before: so does the tile test.
-__device__ __noinline__ bool walk_reaches(int n, const double* aabbs, int i, int j) {
-  const Box a = load_box(aabbs, i), b = load_box(aabbs, j);
+// whose walk no ordered lower x ends before: so does the tile test.  If any
+// box between the two ends the walk, the last ordered one does.
+__device__ __forceinline__ bool walk_reaches(const LastBox& last, const Box& a, int i,
+                                             const Box& b, int j) {
+  if (last.at < 0) return true;
   const bool i_first = comes_first(a, i, b, j);
   const Box& e = i_first ? a : b;  // the earlier of the two in the sweep
   const Box& l = i_first ? b : a;
-  const int ei = i_first ? i : j;
-  if (!(l.lo[0] != l.lo[0]) || e.lo[0] != e.lo[0]) return true;
-  for (int m = 0; m < n; ++m) {
-    const Box c = load_box(aabbs, m);
-    if (c.lo[0] > e.hi[0] && comes_first(e, ei, c, m)) return false;
-  }
-  return true;
+  const int ei = i_first ? i : j, li = i_first ? j : i;
+  Box c{};
+  c.lo[0] = last.lo;
+  return !(last.lo > e.hi[0] && comes_first(e, ei, c, last.at) && comes_first(c, last.at, l, li));
 }
 
 // Rows i0..i0+63 against columns 64 w..64 w + 63: a mask word per row.
@@ -175,12 +202,19 @@ __global__ void __launch_bounds__(256) bp_tiles(int n, int words, const double* 
   const Box b = load_box(aabbs, in ? j : n - 1);
   const int gj = groups ? groups[in ? j : n - 1] : 0;
   unsigned long long mine = 0;
+  LastBox last{0.0, -1};
+  bool have_last = false;
   const int rows = n - i0 < kWave ? n - i0 : kWave;
   for (int r = 0; r < rows; ++r) {
     const int i = i0 + r;
     const Box a = load_box(aabbs, i);
     bool hit = in && j > i && !(groups && groups[i] == gj) && overlap(a, b);
-    if (hit && (a.lo[0] != a.lo[0] || b.lo[0] != b.lo[0])) hit = walk_reaches(n, aabbs, i, j);
+    const bool nan = hit && (a.lo[0] != a.lo[0] || b.lo[0] != b.lo[0]);
+    if (__ballot(nan) != 0) {
+      if (!have_last) last = last_ordered(n, aabbs);
+      have_last = true;
+      if (nan) hit = walk_reaches(last, a, i, b, j);
+    }
     const unsigned long long m = __ballot(hit);
     if (lane == r) mine = m;
   }

@@ -120,3 +120,23 @@ def test_odd_boxes(ctx, seed):
     want = _swept(boxes)
     pairs, num = _run(ctx, boxes, len(want))
     assert num == len(want) and np.array_equal(pairs, want)
+
+
+@pytest.mark.parametrize("n", [64, 65, 700])
+def test_unordered_lower_bounds_of_both_signs(ctx, n):
+    """Negative NaN sorts first and positive NaN last: a walk from the one
+    reaches the other unless an ordered lower x ends it.  Inverted boxes, some
+    of them at the largest lower x."""
+    print("case: broadphase NaN of both signs, n=%d" % n, flush=True)
+    rng = np.random.default_rng(n)
+    boxes = _boxes(n, n, 2.0)
+    boxes[:, 1:3], boxes[:, 4:] = -1, 1  # the x axis decides
+    sign = rng.integers(0, 4, n)
+    boxes[sign == 0, 0] = np.nan
+    boxes[sign == 1, 0] = -np.nan
+    boxes[sign == 3, 3] = rng.choice([np.inf, np.nan, 0.0, -3.0], (sign == 3).sum())
+    boxes[sign == 2, 0] = np.where(rng.random((sign == 2).sum()) < 0.2, 9.0, boxes[sign == 2, 0])
+    want = _swept(boxes)
+    pairs, num = _run(ctx, boxes, len(want) + 3)
+    assert num == len(want) and np.array_equal(pairs[:num], want)
+    assert len(want) < len(_want(boxes))  # some walks end early
