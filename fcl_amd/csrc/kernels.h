@@ -21,6 +21,15 @@ enum : int32_t {
 // host rejects meshes whose summed depths exceed it.
 constexpr int kMaxStack = 256;
 
+// Most blocks of a kernel that takes a wavefront (or part of one) per query:
+// larger batches loop.  HIP refuses a launch of 2^32 threads, and by this
+// size the chip's few thousand wavefront slots have long averaged out the
+// queries' lengths.
+constexpr int kMaxGroupBlocks = 1 << 20;
+inline unsigned group_blocks(long long want) {
+  return static_cast<unsigned>(want < kMaxGroupBlocks ? want : kMaxGroupBlocks);
+}
+
 struct CollideLaunch {
   const MeshDev* meshes;       // device table indexed by mesh id
   int32_t num_meshes;

@@ -87,36 +87,41 @@ constexpr int kSweepLanes = 16;
 __global__ void __launch_bounds__(256) bp_sweep(int n, const Box* boxes, const int32_t* groups,
                                                 const int32_t* sorted, int bits, uint64_t* out,
                                                 long long capacity, unsigned long long* count) {
-  const int k = (blockIdx.x * blockDim.x + threadIdx.x) / kSweepLanes;
   const int lane = threadIdx.x % kWave, first = lane & ~(kSweepLanes - 1);
-  bool live = k < n;
-  const int at = live ? k : n - 1;
-  const Box a = boxes[at];
-  const int i = sorted[at], gi = groups ? groups[at] : 0;
-  for (int m0 = at + 1; __ballot(live) != 0; m0 += kSweepLanes) {
-    const int m = m0 + (lane - first);
-    bool end = m >= n, hit = false;
-    if (live && !end) {
-      const Box b = boxes[m];
-      end = b.lo[0] > a.hi[0];  // sorted by lower x: no later box reaches i
-      hit = !end && !(groups && groups[m] == gi) && overlap(a, b);
-    }
-    // lanes past the first end are past the walk
-    const unsigned ends = static_cast<unsigned>(__ballot(end) >> first) & ((1u << kSweepLanes) - 1);
-    if (ends != 0 && lane - first > __ffs(static_cast<int>(ends)) - 1) hit = false;
-    if (ends != 0) live = false;
-    const unsigned long long hm = __ballot(hit);
-    if (hm == 0) continue;
-    unsigned long long base = 0;
-    const int leader = __ffsll(static_cast<long long>(hm)) - 1;
-    if (lane == leader) base = atomicAdd(count, static_cast<unsigned long long>(__popcll(hm)));
-    base = __shfl(base, leader);
-    if (!hit) continue;
-    const unsigned long long slot = base + __popcll(hm & ((1ULL << lane) - 1ULL));
-    if (static_cast<long long>(slot) < capacity) {
-      const int j = sorted[m];
-      const uint64_t low = static_cast<uint64_t>(i < j ? i : j);
-      out[slot] = (low << bits) | static_cast<uint64_t>(i < j ? j : i);
+  const int step = static_cast<int>(gridDim.x * (blockDim.x / kSweepLanes));
+  // (the last round's wavefronts may hold walks past the last object)
+  long long k = (blockIdx.x * blockDim.x + threadIdx.x) / kSweepLanes;
+  for (; __ballot(k < n) != 0; k += step) {
+    bool live = k < n;
+    const int at = live ? static_cast<int>(k) : n - 1;
+    const Box a = boxes[at];
+    const int i = sorted[at], gi = groups ? groups[at] : 0;
+    for (int m0 = at + 1; __ballot(live) != 0; m0 += kSweepLanes) {
+      const int m = m0 + (lane - first);
+      bool end = m >= n, hit = false;
+      if (live && !end) {
+        const Box b = boxes[m];
+        end = b.lo[0] > a.hi[0];  // sorted by lower x: no later box reaches i
+        hit = !end && !(groups && groups[m] == gi) && overlap(a, b);
+      }
+      // lanes past the first end are past the walk
+      const unsigned ends =
+          static_cast<unsigned>(__ballot(end) >> first) & ((1u << kSweepLanes) - 1);
+      if (ends != 0 && lane - first > __ffs(static_cast<int>(ends)) - 1) hit = false;
+      if (ends != 0) live = false;
+      const unsigned long long hm = __ballot(hit);
+      if (hm == 0) continue;
+      unsigned long long base = 0;
+      const int leader = __ffsll(static_cast<long long>(hm)) - 1;
+      if (lane == leader) base = atomicAdd(count, static_cast<unsigned long long>(__popcll(hm)));
+      base = __shfl(base, leader);
+      if (!hit) continue;
+      const unsigned long long slot = base + __popcll(hm & ((1ULL << lane) - 1ULL));
+      if (static_cast<long long>(slot) < capacity) {
+        const int j = sorted[m];
+        const uint64_t low = static_cast<uint64_t>(i < j ? i : j);
+        out[slot] = (low << bits) | static_cast<uint64_t>(i < j ? j : i);
+      }
     }
   }
 }
@@ -357,8 +362,8 @@ hipError_t run_sweep(int n, const double* aabbs, const int32_t* groups, int32_t*
                                          sorted, n, 0, 64, s);
   if (e == hipSuccess) {
     bp_gather<<<grid, block, 0, s>>>(n, aabbs, groups, sorted, boxes, sorted_groups);
-    bp_sweep<<<static_cast<unsigned>((static_cast<long long>(n) * kSweepLanes + block - 1) / block),
-               block, 0, s>>>(n, boxes, sorted_groups, sorted, bits, pk,
+    bp_sweep<<<group_blocks((static_cast<long long>(n) * kSweepLanes + block - 1) / block), block, 0,
+               s>>>(n, boxes, sorted_groups, sorted, bits, pk,
                               static_cast<long long>(cap), count);
     bp_store_count<<<1, 1, 0, s>>>(count, num_pairs);
     e = hipGetLastError();

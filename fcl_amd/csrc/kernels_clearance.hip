@@ -345,9 +345,25 @@ __global__ void __launch_bounds__(kWave, 1) distance_ordered(DistanceLaunch L, i
 bool distance_ordered_takes(size_t max_nodes) { return max_nodes <= (size_t(1) << kIdBits); }
 
 hipError_t launch_distance_ordered(const DistanceLaunch& L, int stack_need, hipStream_t s) {
-  if (L.num_queries <= 0) return hipSuccess;
-  distance_ordered<<<static_cast<unsigned>(L.num_queries), kWave, 0, s>>>(L, stack_need + 2);
-  return hipGetLastError();
+  // HIP refuses a launch of 2^32 threads: larger batches in parts (a loop in
+  // the kernel took 2 % of a single call)
+  constexpr int kPart = 1 << 25;
+  DistanceLaunch P = L;
+  for (int left = L.num_queries; left > 0; left -= kPart) {
+    P.num_queries = left < kPart ? left : kPart;
+    distance_ordered<<<static_cast<unsigned>(P.num_queries), kWave, 0, s>>>(P, stack_need + 2);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    P.query_meshes += 2 * static_cast<size_t>(kPart);
+    P.tf1 += 12 * static_cast<size_t>(kPart);
+    P.tf2 += 12 * static_cast<size_t>(kPart);
+    P.distance += kPart;
+    if (P.points) P.points += 6 * static_cast<size_t>(kPart);
+    if (P.ids) P.ids += 2 * static_cast<size_t>(kPart);
+    if (P.bv_tests) P.bv_tests += kPart;
+    if (P.leaf_tests) P.leaf_tests += kPart;
+  }
+  return hipSuccess;
 }
 
 }  // namespace fclx

@@ -484,16 +484,13 @@ __device__ __forceinline__ bool leaf_inside(const MsWave& w, const double* tv, d
 // query; 200,000 links that nearly all collide at once 8.3 ms, now 7.3.
 // Quarter wavefronts are faster for the latter (4.2 ms) and slower for the
 // former (28 ms).
-template <bool kStats, bool kContact, int kWaves>
-__global__ void __launch_bounds__(64, kWaves) meshshape_ordered(MeshShapeLaunch L,
-                                                                const MsQuery* queries, int margin,
-                                                                int leaf_min, MsEpaSeed* seeds,
-                                                                unsigned long long* nseed) {
+template <bool kStats, bool kContact>
+__device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery* queries, size_t q,
+                                        int margin, int leaf_min, MsEpaSeed* seeds,
+                                        unsigned long long* nseed,
+                                        OrderedList<kMsListCap, kStats>& S, MsWave& w) {
   constexpr int G = 64, kCap = kMsListCap;
-  __shared__ OrderedList<kCap, kStats> S;
-  __shared__ MsWave w;
   const LaneGroup<G> g;
-  const size_t q = blockIdx.x;
   if (queries[q].valid == 0) return;
   OrdTotals T;
   if (g.lane == 0) {
@@ -633,6 +630,17 @@ __global__ void __launch_bounds__(64, kWaves) meshshape_ordered(MeshShapeLaunch 
       L.stats[2 * q + 1] = T.leaf;
     }
   }
+}
+
+template <bool kStats, bool kContact, int kWaves>
+__global__ void __launch_bounds__(64, kWaves) meshshape_ordered(MeshShapeLaunch L,
+                                                                const MsQuery* queries, int margin,
+                                                                int leaf_min, MsEpaSeed* seeds,
+                                                                unsigned long long* nseed) {
+  __shared__ OrderedList<kMsListCap, kStats> S;
+  __shared__ MsWave w;
+  for (size_t q = blockIdx.x; q < static_cast<size_t>(L.num_queries); q += gridDim.x)
+    descend<kStats, kContact>(L, queries, q, margin, leaf_min, seeds, nseed, S, w);
 }
 
 // Lanes of a wavefront step together: a lane whose descent reached a leaf
@@ -881,8 +889,8 @@ void launch_descent(const MeshShapeLaunch& L, const MsQuery* queries, MsEpaSeed*
                           : (L.stats ? meshshape_ordered<true, false, kWaves>
                                      : meshshape_ordered<false, false, kWaves>);
   const int leaf_min = L.leaf_share > 0 ? std::max(1, 64 * L.leaf_share / 100) : 64;
-  kernel<<<static_cast<unsigned>(L.num_queries), 64, 0, s>>>(L, queries, L.max_depth + 2, leaf_min,
-                                                             seeds, nseed);
+  kernel<<<group_blocks(L.num_queries), 64, 0, s>>>(L, queries, L.max_depth + 2, leaf_min, seeds,
+                                                    nseed);
 }
 
 // Stream-ordered scratch of one batch, freed (in stream order) at its end.

@@ -181,18 +181,18 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
   OrderedList<kCap, kStats>& S = W.list[gi];
   const QueryXf64& x = W.x64[gi];
   int q = -1;  // the group's query; -2: none left
+  unsigned next = blockIdx.x * (kWave / G) + gi;
   OrdTotals T;
-  bool taken = false;
   while (true) {
     // groups without a query take the next one
     const unsigned long long need = __ballot(g.lane == 0 && q == -1);
     if (need != 0) {
       if (q == -1) {
-        const long long next = static_cast<long long>(blockIdx.x) * (kWave / G) + gi;
-        q = !taken && next < L.num_queries ? static_cast<int>(next) : -2;
-        taken = true;
+        q = next < static_cast<unsigned>(L.num_queries) ? static_cast<int>(next) : -2;
+        next += gridDim.x * (kWave / G);
         if (q >= 0) {
-          const int i1 = L.query_meshes[2 * q], i2 = L.query_meshes[2 * q + 1];
+          const int32_t* qm = L.query_meshes + 2 * static_cast<size_t>(q);
+          const int i1 = qm[0], i2 = qm[1];
           if (!obbrss_query_ok(L.meshes, L.num_meshes, i1, i2)) {
             if (g.lane == 0) {
               L.counts[q] = 0;
@@ -314,14 +314,14 @@ hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStr
   if (L.num_queries >= kNarrowMin && L.cap == 1 && !L.contact && !L.bv_tests && !L.leaf_tests &&
       margin + 16 <= list_cap<16>()) {
     collide_ordered<16, false, false>
-        <<<static_cast<unsigned>((L.num_queries + 3LL) / 4), kWave, 0, s>>>(L, margin, 8);
+        <<<group_blocks((L.num_queries + 3LL) / 4), kWave, 0, s>>>(L, margin, 8);
   } else {
     const bool stats = L.bv_tests || L.leaf_tests;
     auto kernel = L.contact
                       ? (stats ? collide_ordered<64, true, true> : collide_ordered<64, false, true>)
                       : (stats ? collide_ordered<64, true, false>
                                : collide_ordered<64, false, false>);
-    kernel<<<static_cast<unsigned>(L.num_queries), kWave, 0, s>>>(L, margin, 16);
+    kernel<<<group_blocks(L.num_queries), kWave, 0, s>>>(L, margin, 16);
   }
   return hipGetLastError();
 }
