@@ -113,6 +113,7 @@ struct fclx_context {
   int epa_blocks_per_cu = 0;
   int shape_waves = 2;
   std::atomic<int> serve_fail_launches{0};  // failure injection for the serving loop
+  std::atomic<uint32_t> ordered_carry_max{1u << 31};
 };
 
 namespace {
@@ -667,6 +668,7 @@ int collide_batch_status(fclx_context* ctx, const fclx_collide_batch_args* a, vo
   L.bv_tests = reinterpret_cast<long long*>(a->bv_tests);
   L.leaf_tests = reinterpret_cast<long long*>(a->leaf_tests);
   L.status = d_status;
+  L.carry_max = ctx->ordered_carry_max.load();
   hipError_t e;
   if (a->enable_contact) {
     // contact geometry follows the reference's order and per-contact cap
@@ -888,6 +890,7 @@ int fclx_mesh_shape_collide_batch(fclx_context* ctx, const fclx_mesh_shape_colli
   L.contact_depth = a->contact_depth;
   L.stats = reinterpret_cast<long long*>(a->stats);
   L.status = ctx->d_status;
+  L.carry_max = ctx->ordered_carry_max.load();
   int waves;
   {
     std::lock_guard<std::mutex> lock(ctx->ws_mu);
@@ -1060,6 +1063,7 @@ int fclx_get_engine_param(fclx_context* ctx, const char* name, double* value) {
   else if (n == "dist_waves_per_simd") *value = t.dist.waves_per_simd;
   else if (n == "meshshape_waves_per_simd") *value = t.meshshape_waves_per_simd;
   else if (n == "meshshape_leaf_share") *value = t.meshshape_leaf_share;
+  else if (n == "ordered_carry_max") *value = ctx->ordered_carry_max.load();
   else if (n == "dist_width") *value = t.dist.width;
   else if (n == "dist_leaf_batch") *value = t.dist.leaf_batch;
   else if (n == "dist_fp32_cull") *value = t.dist.fp32_cull;
@@ -1116,6 +1120,8 @@ int fclx_set_engine_param(fclx_context* ctx, const char* name, double value) {
     t.meshshape_waves_per_simd = static_cast<int>(value);
   } else if (n == "meshshape_leaf_share" && in(0, 100)) {
     t.meshshape_leaf_share = static_cast<int>(value);
+  } else if (n == "ordered_carry_max" && in(1, 1LL << 31)) {
+    ctx->ordered_carry_max.store(static_cast<uint32_t>(value));
   } else if (n == "dist_width" && in(1, 64)) {
     t.dist.width = static_cast<int>(value);
   } else if (n == "dist_leaf_batch" && in(1, 64)) {
@@ -1414,6 +1420,7 @@ int collide_one(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_t 
     L.bv_tests = io.tests;
     L.leaf_tests = io.tests + 1;
     L.status = ctx->s_status;
+    L.carry_max = ctx->ordered_carry_max.load();
     if (contact) {
       L.contact = 1;
       L.contact_pos = ctx->s_geo;

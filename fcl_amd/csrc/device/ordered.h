@@ -15,7 +15,11 @@
 // Test counts: every entry carries the tests already done on nodes that lie
 // before it in visit order and after the entry before it.  An entry that
 // vanishes hands its tests to the next one; dropped entries take theirs
-// along.  The sums are exactly the recursion's counts.
+// along.  The sums are exactly the recursion's counts.  Entries carry 32
+// bits, totals 64: before the list can carry carry_max tests (2^31 unless set
+// lower) ord_audit counts the top entry's, which lie before anything that can
+// still be dropped, and has the group take one entry at a time while the list
+// carries too many.
 //
 // Stack bound: a step that takes n entries grows the list by at most n.  A
 // group takes no more than the room left above a margin of one tree path,
@@ -94,6 +98,10 @@ template <int kCap, bool kStats>
 struct OrderedList {
   unsigned long long e[kCap];
   uint2 acc[kStats ? kCap : 1];
+  // The query's BV (x) and leaf (y) tests up to the last commit and behind
+  // the last entry, kept by lane 0 (here rather than in registers, which the
+  // kernels are short of).
+  longlong2 total, tail;
 };
 
 // What a step made of this lane's entry (lanes past the step's window: none).
@@ -105,13 +113,29 @@ struct OrdOutcome {
   unsigned bv = 0, leaf = 0;   // tests done on it in this step
 };
 
-// Traversal totals of a group's query (the same values in all its lanes).
+// State of a group's query (the same values in all its lanes).
 struct OrdTotals {
   int sp = 0;
-  int count = 0;               // contacts committed
-  long long bv = 0, leaf = 0;  // tests up to the last commit
-  long long tail_bv = 0, tail_leaf = 0;  // tests behind the last entry of the list
+  int count = 0;     // contacts committed
+  int audit_in = 0;  // steps before the next ord_audit
 };
+
+// A query's list with the root in it.
+template <int G, int kCap, bool kStats>
+__device__ __forceinline__ OrdTotals ord_begin(const LaneGroup<G>& g, OrderedList<kCap, kStats>& S,
+                                               unsigned carry_max) {
+  OrdTotals W;
+  W.sp = 1;
+  W.audit_in = static_cast<int>(carry_max / 128);
+  if (g.lane == 0) {
+    S.e[0] = ord_pack(kOrdNode, 0, 0);
+    if constexpr (kStats) {
+      S.acc[0] = make_uint2(0u, 0u);
+      S.total = S.tail = make_longlong2(0, 0);
+    }
+  }
+  return W;
+}
 
 // Entries the group takes from the top of its list in a step.
 template <int G, int kCap>
@@ -120,6 +144,30 @@ __device__ __forceinline__ int ord_window(int sp, int margin) {
   int n = sp < G ? sp : G;
   if (n > room) n = room > 1 ? room : 1;
   return n;
+}
+
+// Before a step's window of n entries is read, once audit_in steps are over
+// (adding the top's tests to the totals in each step took 3 % of a single
+// call).  A list that carries less than half of carry_max goes on for as many
+// full steps as cannot add the other half (64 tests each); else the step takes
+// the top entry alone, whose tests reach the totals in the next one.  Either
+// way no entry comes to carry more than carry_max + 64.
+template <int G, int kCap>
+__device__ __forceinline__ void ord_audit(const LaneGroup<G>& g, OrderedList<kCap, true>& S,
+                                          OrdTotals& W, unsigned carry_max, int& n) {
+  if (g.lane == 0 && n > 0) {
+    const uint2 top = S.acc[W.sp - 1];
+    S.total = make_longlong2(S.total.x + top.x, S.total.y + top.y);
+    S.acc[W.sp - 1] = make_uint2(0u, 0u);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  unsigned sum = 0;  // (carries below 2^32 in all)
+  for (int k = g.lane; k < W.sp; k += G) sum += S.acc[k].x;
+#pragma unroll
+  for (int d = 1; d < G; d <<= 1) sum += __shfl_xor(sum, d);
+  const bool many = sum >= carry_max / 2;
+  if (many && n > 1) n = 1;
+  W.audit_in = many ? 0 : static_cast<int>(carry_max / 128);
 }
 
 // Puts a step's outcomes back.  Leading hits are committed: emit(mine,
@@ -149,7 +197,8 @@ __device__ __forceinline__ void ord_settle(const LaneGroup<G>& g, OrderedList<kC
     if (reach != 0) {
       last = __ffsll(static_cast<long long>(reach)) - 1;
       base = 0;
-      W.tail_bv = W.tail_leaf = 0;
+      if constexpr (kStats)
+        if (g.lane == 0) S.tail = make_longlong2(0, 0);
       if (g.lane > last) nout = 0;
     }
     const unsigned long long open = g.ballot(nout > 0 && !hit);
@@ -191,27 +240,22 @@ __device__ __forceinline__ void ord_settle(const LaneGroup<G>& g, OrderedList<kC
     const unsigned tl = g.at(pl, G - 1) - (end < 0 ? 0u : el);
     const unsigned cb = g.at(pb, committed < 0 ? 0 : committed);
     const unsigned cl = g.at(pl, committed < 0 ? 0 : committed);
-    if (committed >= 0) {
-      W.bv += cb;
-      W.leaf += cl;
-    }
-    if (base > 0) {
-      if (g.lane == 0 && n > 0) {
+    if (g.lane == 0 && n > 0) {
+      if (committed >= 0) S.total = make_longlong2(S.total.x + cb, S.total.y + cl);
+      if (base > 0) {
         const uint2 a = S.acc[base - 1];
         S.acc[base - 1] = make_uint2(a.x + tb, a.y + tl);
+      } else {
+        S.tail = make_longlong2(S.tail.x + tb, S.tail.y + tl);
       }
-    } else {
-      W.tail_bv += tb;
-      W.tail_leaf += tl;
     }
   }
   W.sp = sp;
   if (n > 0 && (sp == 0 || W.count >= cap)) {
     W.sp = 0;
-    if (W.count < cap) {  // the whole tree was visited
-      W.bv += W.tail_bv;
-      W.leaf += W.tail_leaf;
-    }
+    if constexpr (kStats)  // below the cap the whole tree was visited
+      if (g.lane == 0 && W.count < cap)
+        S.total = make_longlong2(S.total.x + S.tail.x, S.total.y + S.tail.y);
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }

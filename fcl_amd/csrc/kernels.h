@@ -49,6 +49,7 @@ struct CollideLaunch {
   // enable_contact (plain kernel only): a record per contact, with its
   // world-frame point (3), normal (3) and penetration depth
   int32_t contact;
+  uint32_t carry_max;          // ordered kernel: most BV tests its list carries
   double* contact_pos;
   double* contact_normal;
   double* contact_depth;
@@ -115,6 +116,7 @@ struct MeshShapeLaunch {
   int32_t* status;
   int32_t leaf_share;           // percent of a wavefront's lanes with a leaf that starts a
                                 // leaf round (1..100; 0: 100)
+  uint32_t carry_max;           // most BV tests that a query's list carries
   int32_t max_depth;            // deepest mesh of the context (levels)
 };
 // waves: register budget, 1..3 waves per SIMD

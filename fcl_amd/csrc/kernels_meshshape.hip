@@ -492,7 +492,7 @@ __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery*
   constexpr int G = 64, kCap = kMsListCap;
   const LaneGroup<G> g;
   if (queries[q].valid == 0) return;
-  OrdTotals T;
+  OrdTotals T = ord_begin(g, S, L.carry_max);
   if (g.lane == 0) {
     const MeshDev& M = L.meshes[L.query_meshes[q]];
     (void)load_query(L, static_cast<int>(q), w.s, L.max_depth);
@@ -519,13 +519,12 @@ __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery*
     w.n32 = M.obb32;
     w.n64 = M.obb64;
     w.tris = M.tri_verts;
-    S.e[0] = ord_pack(kOrdNode, 0, 0);
-    if constexpr (kStats) S.acc[0] = make_uint2(0u, 0u);
   }
-  T.sp = 1;
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   while (T.sp > 0) {
-    const int n = ord_window<G, kCap>(T.sp, margin);
+    int n = ord_window<G, kCap>(T.sp, margin);
+    if constexpr (kStats)
+      if (--T.audit_in < 0) ord_audit(g, S, T, L.carry_max, n);
     const bool on = g.lane < n;
     unsigned long long e = 0;
     uint2 acc = make_uint2(0u, 0u);
@@ -626,8 +625,8 @@ __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery*
   if (g.lane == 0) {
     L.counts[q] = T.count;
     if constexpr (kStats) {
-      L.stats[2 * q] = T.bv;
-      L.stats[2 * q + 1] = T.leaf;
+      L.stats[2 * q] = S.total.x;
+      L.stats[2 * q + 1] = S.total.y;
     }
   }
 }

@@ -227,11 +227,8 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
               W.x64[gi] = y;
               W.x32[gi] = X;
               W.ptr[gi] = QueryPtr{m1.obb32, m2.obb32, m1.size64, m2.size64};
-              S.e[0] = ord_pack(kOrdNode, 0, 0);
-              if constexpr (kStats) S.acc[0] = make_uint2(0u, 0u);
             }
-            T = OrdTotals();
-            T.sp = 1;
+            T = ord_begin(g, S, L.carry_max);
           }
         }
       }
@@ -239,7 +236,9 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
     }
     if (__ballot(q != -2) == 0) break;
     // the window: lane k holds the list's entry k from the top
-    const int n = q >= 0 ? ord_window<G, kCap>(T.sp, margin) : 0;
+    int n = q >= 0 ? ord_window<G, kCap>(T.sp, margin) : 0;
+    if constexpr (kStats)
+      if (__ballot(--T.audit_in < 0) != 0) ord_audit(g, S, T, L.carry_max, n);
     const bool on = g.lane < n;
     unsigned long long e = 0;
     uint2 acc = make_uint2(0u, 0u);
@@ -296,8 +295,8 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
       if (g.lane == 0) {
         L.counts[q] = T.count;
         if constexpr (kStats) {
-          if (L.bv_tests) L.bv_tests[q] = T.bv;
-          if (L.leaf_tests) L.leaf_tests[q] = T.leaf;
+          if (L.bv_tests) L.bv_tests[q] = S.total.x;
+          if (L.leaf_tests) L.leaf_tests[q] = S.total.y;
         }
       }
       q = -1;

@@ -400,6 +400,10 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               to test that starts their leaf tests
  *                               (default 0: 100, or when nothing else is
  *                               left to test)
+ *   "ordered_carry_max" 1..2^31 test counts that the traversals in the
+ *                               reference's order hold ahead of their turn
+ *                               before they go one node at a time (default
+ *                               2^31: counts are 64-bit throughout)
  *   "dist_width"        1..64   most bounds of one query per distance step
  *                               (default 32)
  *   "dist_leaf_batch"   1..64   leaf pairs queued before their distances are

@@ -115,3 +115,21 @@ def test_sizes_at_the_ends_of_floats(scale):
         assert np.array_equal(pairs, want[2].get(q, np.zeros((0, 2))))
         assert stats.tolist() == [want[3][q], want[4][q]]
     local.close()
+
+
+@pytest.mark.parametrize("carry_max", [1, 9, 300])
+def test_counts_at_the_carry_limit(pair, ctx, carry_max):
+    """Test counts are summed in 64 bits, whatever the list may carry ahead."""
+    n = 200
+    print("case: ordered groups, carry limit %d" % carry_max, flush=True)
+    tf1, tf2 = F.poses(n, 0, 1.7, 0, 0xCA)
+    qm = np.tile(np.array(pair, np.int32), (n, 1))
+    ctx.set_engine_param("ordered_carry_max", carry_max)
+    try:
+        for cap in (1, 3, 64):
+            want = _same(ctx, qm, tf1, tf2, cap, True)
+        _, stats = ctx.collide(pair[0], tf1[5], pair[1], tf2[5], cap=64)
+        assert stats.tolist() == [want[3][5], want[4][5]]
+    finally:
+        ctx.set_engine_param("ordered_carry_max", 2**31)
+    assert ctx.get_engine_param("ordered_carry_max") == 2**31

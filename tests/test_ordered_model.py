@@ -54,7 +54,9 @@ def recursion(tree, cap):
 class Group:
     """One group's query: the list (top last), totals, the records emitted."""
 
-    def __init__(self, tree, cap, G, list_cap, margin, mistake=None):
+    def __init__(self, tree, cap, G, list_cap, margin, mistake=None, carry_max=2**31):
+        self.carry_max, self.most, self.serial = carry_max, 0, 0
+        self.audit_in = carry_max // 128
         self.tree, self.cap, self.G = tree, cap, G
         self.list_cap, self.margin, self.mistake = list_cap, margin, mistake
         self.e, self.acc = [(NODE, "")], [[0, 0]]
@@ -67,8 +69,20 @@ class Group:
         n = min(len(self.e), self.G)
         return n if n <= room else max(room, 1)
 
+    def audit(self):
+        self.bv += self.acc[-1][0]
+        self.leaf += self.acc[-1][1]
+        self.acc[-1] = [0, 0]
+        many = sum(a[0] for a in self.acc) >= self.carry_max // 2
+        self.audit_in = 0 if many else self.carry_max // 128
+        self.serial += many
+        return many
+
     def step(self, test_leaves):
         n = self.window()
+        self.audit_in -= 1
+        if self.audit_in < 0 and self.audit():
+            n = 1
         lanes = [(self.e[-1 - k], self.acc[-1 - k]) for k in range(n)]
         base = len(self.e) - n
         nodes = sum(e[0] == NODE for e, _ in lanes)
@@ -144,6 +158,7 @@ class Group:
             self.tail = [self.tail[j] + rest[j] for j in (0, 1)]
         self.e += new_e[::-1]
         self.acc = below + new_acc[::-1]
+        self.most = max([self.most] + [x for a in self.acc for x in a])
         self.high = max(self.high, len(self.e))
         self.steps += 1
         if not self.e or self.count >= self.cap:
@@ -178,6 +193,24 @@ def test_group_traversal_is_the_recursion(G, list_cap, contact):
             narrow += g.high > list_cap - depth - 3
             ended += len(want[0]) == cap
     assert ended > 20 and (narrow > 0 or list_cap > 100)
+
+
+@pytest.mark.parametrize("carry_max", [1, 40, 300])
+def test_no_entry_carries_more_than_its_bits(carry_max):
+    """A list near its carry limit goes one node at a time: same answers and
+    counts, and no entry carries more than the limit and one step's tests."""
+    rng = random.Random(carry_max)
+    G, free, held = 64, 0, 0
+    for seed in range(25):
+        tree = Tree(seed, rng.randint(6, 13), 0.85, rng.choice([0.0, 0.05]), False)
+        for cap in (1, 7, 10**6):
+            want = recursion(tree, cap)
+            g = Group(tree, cap, G, 512, 16, carry_max=carry_max)
+            assert g.run(rng) == want and g.most <= carry_max + G
+            u = Group(tree, cap, G, 512, 16)
+            assert u.run(rng) == want
+            free, held = max(free, u.most), held + (g.serial > 0)
+    assert free > carry_max + G and held > 5
 
 
 def test_a_planted_mistake_is_seen():
