@@ -114,6 +114,7 @@ struct fclx_context {
   int shape_waves = 2;
   std::atomic<int> serve_fail_launches{0};  // failure injection for the serving loop
   std::atomic<uint32_t> ordered_carry_max{1u << 31};
+  std::atomic<int> ordered_lanes{0};
 };
 
 namespace {
@@ -191,6 +192,19 @@ size_t max_nodes(const fclx_context* ctx) {
   for (const auto& m : ctx->meshes)
     if (m.live) n = std::max(n, m.bvh.nodes.size());
   return n;
+}
+
+size_t min_nodes(const fclx_context* ctx) {
+  size_t n = 0;
+  for (const auto& m : ctx->meshes)
+    if (m.live) n = n == 0 ? m.bvh.nodes.size() : std::min(n, m.bvh.nodes.size());
+  return n;
+}
+
+// lanes_max of a batch under the "ordered_lanes" tunable: the rule's, none or all.
+long long lanes_max(const fclx_context* ctx, long long rule) {
+  const int mode = ctx->ordered_lanes.load();
+  return mode == 0 ? rule : (mode == 1 ? 0 : kAllLanes);
 }
 
 // The FAST engine packs (query, node, node) into 64 bits: 21 bits per node.
@@ -640,12 +654,13 @@ int collide_batch_status(fclx_context* ctx, const fclx_collide_batch_args* a, vo
     return fail(ctx, FCLX_ERR_INVALID_ARGUMENT, "invalid collide batch arguments");
   hipStream_t s = static_cast<hipStream_t>(stream);
   int depth, nmesh;
-  size_t nodes;
+  size_t nodes, nodes_min;
   const MeshDev* table;
   {
     std::lock_guard<std::mutex> lock(ctx->mu);
     depth = max_depth(ctx);
     nodes = max_nodes(ctx);
+    nodes_min = min_nodes(ctx);
     nmesh = static_cast<int>(ctx->meshes.size());
     table = ctx->d_table;
   }
@@ -669,6 +684,8 @@ int collide_batch_status(fclx_context* ctx, const fclx_collide_batch_args* a, vo
   L.leaf_tests = reinterpret_cast<long long*>(a->leaf_tests);
   L.status = d_status;
   L.carry_max = ctx->ordered_carry_max.load();
+  L.lanes_max = lanes_max(ctx, collide_lanes_max(a->num_queries, a->num_max_contacts, nodes_min,
+                                                 nodes));
   hipError_t e;
   if (a->enable_contact) {
     // contact geometry follows the reference's order and per-contact cap
@@ -1064,6 +1081,7 @@ int fclx_get_engine_param(fclx_context* ctx, const char* name, double* value) {
   else if (n == "meshshape_waves_per_simd") *value = t.meshshape_waves_per_simd;
   else if (n == "meshshape_leaf_share") *value = t.meshshape_leaf_share;
   else if (n == "ordered_carry_max") *value = ctx->ordered_carry_max.load();
+  else if (n == "ordered_lanes") *value = ctx->ordered_lanes.load();
   else if (n == "dist_width") *value = t.dist.width;
   else if (n == "dist_leaf_batch") *value = t.dist.leaf_batch;
   else if (n == "dist_fp32_cull") *value = t.dist.fp32_cull;
@@ -1122,6 +1140,8 @@ int fclx_set_engine_param(fclx_context* ctx, const char* name, double value) {
     t.meshshape_leaf_share = static_cast<int>(value);
   } else if (n == "ordered_carry_max" && in(1, 1LL << 31)) {
     ctx->ordered_carry_max.store(static_cast<uint32_t>(value));
+  } else if (n == "ordered_lanes" && (value == 0 || value == 1 || value == 2)) {
+    ctx->ordered_lanes.store(static_cast<int>(value));
   } else if (n == "dist_width" && in(1, 64)) {
     t.dist.width = static_cast<int>(value);
   } else if (n == "dist_leaf_batch" && in(1, 64)) {

@@ -62,6 +62,20 @@ __device__ __forceinline__ void make_xf32(const double* R, const double* T, doub
                             (1.0 + 1.0 / 1048576.0));
 }
 
+// The same for a query whose poses may be any matrices: the cull's margin
+// holds for rotations, with any other matrix every test is left to FP64.
+__device__ __forceinline__ void make_xf32_checked(const double* R, const double* T, double cmax1,
+                                                  double cmax2, QueryXf32& X) {
+  make_xf32(R, T, cmax1, cmax2, X);
+  int unit = 1;  // (without branches)
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    unit &= static_cast<int>(sq(col(R, k)) < 1.0001);
+    unit &= static_cast<int>(sq(v3(R[3 * k], R[3 * k + 1], R[3 * k + 2])) < 1.0001);
+  }
+  if (unit == 0) X.ms = INFINITY;
+}
+
 // firstOverSecond's size comparison (bvh_collision_traversal_node-inl.h:
 // 77-89; OBBRSS::size = |OBB extents|^2, OBB-inl.h:206-209) from the FP32
 // extents already loaded with the nodes.  Each FP32 sum of squares is

@@ -46,14 +46,29 @@ struct CollideLaunch {
   long long* bv_tests;         // optional, per query
   long long* leaf_tests;       // optional, per query
   int32_t* status;             // device status word (kStatus* bits)
-  // enable_contact (plain kernel only): a record per contact, with its
+  // enable_contact (not in the plain engine): a record per contact, with its
   // world-frame point (3), normal (3) and penetration depth
   int32_t contact;
   uint32_t carry_max;          // ordered kernel: most BV tests its list carries
   double* contact_pos;
   double* contact_normal;
   double* contact_depth;
+  // Queries of at most this many node pairs (the product of the meshes' node
+  // counts) run on a lane each, the others on lane groups: none, some of the
+  // batch, or kAllLanes
+  long long lanes_max;
 };
+constexpr long long kAllLanes = 0x7fffffffffffffffLL;
+__device__ __forceinline__ long long node_pairs(const MeshDev& a, const MeshDev& b) {
+  return static_cast<long long>(a.num_bvs) * b.num_bvs;
+}
+// lanes_max for a batch of a context whose meshes have from nodes_min to
+// nodes_max nodes: limit, or what it comes to there.
+inline long long lanes_within(long long limit, size_t nodes_min, size_t nodes_max) {
+  if (static_cast<double>(nodes_min) * nodes_min > static_cast<double>(limit)) return 0;
+  if (static_cast<double>(nodes_max) * nodes_max <= static_cast<double>(limit)) return kAllLanes;
+  return limit;
+}
 
 struct DistanceLaunch {
   const MeshDev* meshes;
@@ -124,6 +139,11 @@ hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& L, int waves, hipStr
 size_t mesh_shape_epa_lane_bytes();
 
 hipError_t launch_collide_plain(const CollideLaunch& L, int stack_need, hipStream_t s);
+// a query per lane with FP32 culls, for the queries of L.lanes_max node pairs
+// at most (with contact geometry on request)
+hipError_t launch_collide_lanes(const CollideLaunch& L, int stack_need, hipStream_t s);
+// lanes_max of a batch (kernels_ordered.hip)
+long long collide_lanes_max(int num_queries, int cap, size_t nodes_min, size_t nodes_max);
 // collide() in the reference's order by lane groups, any num_max_contacts,
 // with contact geometry and statistics on request (kernels_ordered.hip)
 hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStream_t s);

@@ -17,6 +17,9 @@
 // geometry 9.4 -> 0.26 ms; one collide() call 440 -> 140 us.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "device/ordered.h"
 #include "device/query32.h"
 #include "kernels.h"
@@ -38,9 +41,11 @@ constexpr int list_cap() {
 // wavefront: the chip is full either way, and a group of 16 tests less ahead
 // of a query's answer.  1,000,000 queries of 2 x 2,420 triangles 15.5 ms by
 // whole wavefronts, 8.7 ms by quarters; 10,000 queries 0.23 against 0.37 ms.
-// With more contacts or geometry (100,000 queries, 8 contacts: 2.3 against
-// 3.9 ms) or statistics (2 x 20,480 triangles: 4.7 against 6.9 ms) little is
-// tested in vain, and whole wavefronts stay ahead.
+// With statistics 65,536 queries 1.31 against 1.21 and 250,000 4.7 against
+// 3.6 ms, with geometry 1.37 against 1.02 and 5.0 against 3.1 (2 x 80
+// triangles, 1,000,000: 11.7 against 6.9 and 13.1 against 6.9).  With more
+// contacts little is tested in vain, and whole wavefronts stay ahead (100,000
+// queries, 8 contacts: 2.3 against 3.9 ms).
 constexpr int kNarrowMin = 65536;
 
 // The FP64 test of a node pair the cull left unsure.
@@ -170,10 +175,14 @@ struct OrderedWave {
 
 // One wavefront per block, one query per group.  leaf_min: gathered leaf
 // pairs of the wavefront that start their triangle tests (a group with
-// nothing else to test starts them too).
-template <int G, bool kStats, bool kContact>
-__global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int margin,
-                                                            int leaf_min) {
+// nothing else to test starts them too).  kSome: queries of L.lanes_max node
+// pairs at most (and those with bad ids) are left to launch_collide_lanes; a
+// wavefront looks through `chunk` queries at a time for the others.  (With
+// statistics the lists of four quarters leave LDS for three wavefronts per
+// SIMD.)
+template <int G, bool kStats, bool kContact, bool kSome>
+__global__ void __launch_bounds__(kWave, G == 16 && kStats ? 3 : 4)
+    collide_ordered(CollideLaunch L, int margin, int leaf_min, int chunk) {
   constexpr int kCap = list_cap<G>();
   __shared__ OrderedWave<G, kStats, kContact> W;
   const LaneGroup<G> g;
@@ -181,15 +190,39 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
   OrderedList<kCap, kStats>& S = W.list[gi];
   const QueryXf64& x = W.x64[gi];
   int q = -1;  // the group's query; -2: none left
-  unsigned next = blockIdx.x * (kWave / G) + gi;
+  unsigned next = blockIdx.x * (kSome ? chunk : kWave / G) + (kSome ? 0 : gi);
+  unsigned from = 0;            // kSome: the chunk looked through
+  unsigned long long todo = 0;  // and its queries left
   OrdTotals T;
   while (true) {
     // groups without a query take the next one
     const unsigned long long need = __ballot(g.lane == 0 && q == -1);
     if (need != 0) {
+      if constexpr (kSome) {
+        while (todo == 0 && next < static_cast<unsigned>(L.num_queries)) {
+          from = next;
+          next += gridDim.x * chunk;
+          const unsigned c = from + __lane_id();
+          bool heavy = static_cast<int>(__lane_id()) < chunk &&
+                       c < static_cast<unsigned>(L.num_queries);
+          if (heavy) {
+            const int32_t* qm = L.query_meshes + 2 * static_cast<size_t>(c);
+            heavy = obbrss_query_ok(L.meshes, L.num_meshes, qm[0], qm[1]) &&
+                    node_pairs(L.meshes[qm[0]], L.meshes[qm[1]]) > L.lanes_max;
+          }
+          todo = __ballot(heavy);
+        }
+      }
       if (q == -1) {
-        q = next < static_cast<unsigned>(L.num_queries) ? static_cast<int>(next) : -2;
-        next += gridDim.x * (kWave / G);
+        if constexpr (kSome) {
+          unsigned long long m = todo;
+          for (int k = __popcll(need & ((1ULL << g.first) - 1ULL)); k > 0; --k) m &= m - 1;
+          q = m != 0 ? static_cast<int>(from) + __ffsll(static_cast<long long>(m)) - 1
+                     : (next < static_cast<unsigned>(L.num_queries) ? -1 : -2);
+        } else {
+          q = next < static_cast<unsigned>(L.num_queries) ? static_cast<int>(next) : -2;
+          next += gridDim.x * (kWave / G);
+        }
         if (q >= 0) {
           const int32_t* qm = L.query_meshes + 2 * static_cast<size_t>(q);
           const int i1 = qm[0], i2 = qm[1];
@@ -210,16 +243,7 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
             y.tv1 = m1.tri_verts;
             y.tv2 = m2.tri_verts;
             QueryXf32 X;
-            make_xf32(y.R, y.T, m1.cmax, m2.cmax, X);
-            // the cull's margin holds for rotations; with any other matrix
-            // every test is left to FP64
-            bool unit = true;
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-              const V3 c = col(y.R, k), w = v3(y.R[3 * k], y.R[3 * k + 1], y.R[3 * k + 2]);
-              unit = unit && sq(c) < 1.0001 && sq(w) < 1.0001;
-            }
-            if (!unit) X.ms = INFINITY;
+            make_xf32_checked(y.R, y.T, m1.cmax, m2.cmax, X);
             X.m1 = i1;
             X.m2 = i2;
             X.valid = 1;
@@ -232,6 +256,8 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
           }
         }
       }
+      if constexpr (kSome)
+        for (int k = __popcll(need); k > 0 && todo != 0; --k) todo &= todo - 1;
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
     if (__ballot(q != -2) == 0) break;
@@ -306,22 +332,51 @@ __global__ void __launch_bounds__(kWave, 4) collide_ordered(CollideLaunch L, int
 
 }  // namespace
 
+// Where a lane per query is the faster form: queries too light to fill a
+// wavefront's steps, in batches large enough to fill the chip's lanes.
+// Measured (lanes / groups): two triangles, 1,000 queries 29 / 33 us and
+// 1,000,000 0.23 / 1.64 ms; a triangle and a box of 12, 16,000 queries to the
+// first contact 160 / 124 us, 65,536 184 / 227, 1,000,000 to 8 contacts 2.4 /
+// 5.1 ms; two boxes to the first contact 65,536 0.41 / 0.39, 250,000 1.1 / 1.3
+// and 1,000,000 3.4 / 5.0 ms, to 8 contacts 12.6 / 10.4; two meshes of 20
+// triangles to the first contact, 1,000,000 6.2 / 5.8.
+long long collide_lanes_max(int num_queries, int cap, size_t nodes_min, size_t nodes_max) {
+  const long long limit =
+      num_queries >= 131072 && cap == 1
+          ? 1024
+          : (num_queries >= 32768 ? 32 : (num_queries >= 512 ? 1 : 0));
+  return lanes_within(limit, nodes_min, nodes_max);
+}
+
 hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStream_t s) {
   if (L.num_queries <= 0) return hipSuccess;
-  const int margin = stack_need + 2;
-  // (a quarter's list must hold a tree path and a step)
-  if (L.num_queries >= kNarrowMin && L.cap == 1 && !L.contact && !L.bv_tests && !L.leaf_tests &&
-      margin + 16 <= list_cap<16>()) {
-    collide_ordered<16, false, false>
-        <<<group_blocks((L.num_queries + 3LL) / 4), kWave, 0, s>>>(L, margin, 8);
-  } else {
-    const bool stats = L.bv_tests || L.leaf_tests;
-    auto kernel = L.contact
-                      ? (stats ? collide_ordered<64, true, true> : collide_ordered<64, false, true>)
-                      : (stats ? collide_ordered<64, true, false>
-                               : collide_ordered<64, false, false>);
-    kernel<<<group_blocks(L.num_queries), kWave, 0, s>>>(L, margin, 16);
+  if (L.lanes_max > 0) {
+    const hipError_t e = launch_collide_lanes(L, stack_need, s);
+    if (e != hipSuccess || L.lanes_max == kAllLanes) return e;
   }
+  const int margin = stack_need + 2;
+  const bool stats = L.bv_tests || L.leaf_tests;
+  // (a quarter's list must hold a tree path and a step)
+  const bool narrow = L.num_queries >= kNarrowMin && L.cap == 1 && margin + 16 <= list_cap<16>();
+  const int G = narrow ? 16 : kWave;
+  auto pick = [&](auto g, auto some) {
+    constexpr int kG = decltype(g)::value;
+    constexpr bool kSome = decltype(some)::value;
+    return L.contact ? (stats ? collide_ordered<kG, true, true, kSome>
+                              : collide_ordered<kG, false, true, kSome>)
+                     : (stats ? collide_ordered<kG, true, false, kSome>
+                              : collide_ordered<kG, false, false, kSome>);
+  };
+  const std::integral_constant<int, 16> quarter;
+  const std::integral_constant<int, 64> whole;
+  const std::true_type some;
+  const std::false_type all;
+  auto kernel = L.lanes_max > 0 ? (narrow ? pick(quarter, some) : pick(whole, some))
+                                : (narrow ? pick(quarter, all) : pick(whole, all));
+  // a wavefront's queries to look through: few enough to leave all busy
+  const int chunk = L.lanes_max > 0 ? std::min(std::max(L.num_queries / 8192, 1), kWave) : kWave / G;
+  kernel<<<group_blocks((L.num_queries + chunk - 1LL) / chunk), kWave, 0, s>>>(
+      L, margin, narrow ? 8 : 16, chunk);
   return hipGetLastError();
 }
 

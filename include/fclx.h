@@ -404,6 +404,9 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               reference's order hold ahead of their turn
  *                               before they go one node at a time (default
  *                               2^31: counts are 64-bit throughout)
+ *   "ordered_lanes"     0..2    traversals in the reference's order: a lane per
+ *                               query for light queries in large batches
+ *                               (0, default), for none (1), for all (2)
  *   "dist_width"        1..64   most bounds of one query per distance step
  *                               (default 32)
  *   "dist_leaf_batch"   1..64   leaf pairs queued before their distances are

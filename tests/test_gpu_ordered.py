@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import fcl_amd as F
+from fcl_amd import workloads as W
 from test_gpu_parity import _t, collide_gpu
 
 pytestmark = pytest.mark.gpu
@@ -133,3 +134,63 @@ def test_counts_at_the_carry_limit(pair, ctx, carry_max):
     finally:
         ctx.set_engine_param("ordered_carry_max", 2**31)
     assert ctx.get_engine_param("ordered_carry_max") == 2**31
+
+
+TRIANGLE = np.array([[0.9, 0, 0], [-0.4, 0.8, 0], [-0.4, -0.8, 0.1]]), np.array([[0, 1, 2]])
+BOX = W.box_mesh(np.zeros(3), np.array([1.0, 1.1, 0.9]), 0.3)
+
+
+def _answers(local, m, n, cap, contact, seed=5):
+    tf1, tf2 = F.poses(n, 0, 1.4, 0, seed)
+    counts = torch.full((n,), -1, dtype=torch.int32, device=DEV)
+    num = torch.zeros(1, dtype=torch.int64, device=DEV)
+    rows = n * min(cap, 12)
+    pairs = torch.full((rows, 3), n, dtype=torch.int32, device=DEV)
+    geo = [torch.zeros((rows,) + k, dtype=torch.float64, device=DEV) for k in ((3,), (3,), ())]
+    tests = [torch.full((n,), -1, dtype=torch.int64, device=DEV) for _ in range(2)]
+    s = torch.cuda.current_stream().cuda_stream
+    local.collide_batch_async(_t(m, torch.int32), _t(tf1, torch.float64), _t(tf2, torch.float64),
+                              cap, counts, pairs, num, engine=F.ENGINE_FAST, bv_tests=tests[0],
+                              leaf_tests=tests[1], contact=geo if contact else None, stream=s)
+    rc = local.sync_status(s)
+    order = torch.argsort(pairs[:, 0], stable=True)
+    return rc, [t.cpu().numpy() for t in [counts, num] + tests + [pairs[order]] +
+                [g[order] for g in geo]]
+
+
+@pytest.mark.parametrize("cap,contact", [(1, False), (3, False), (1, True), (4, True)])
+@pytest.mark.parametrize("mode", [0, 2])
+def test_lanes_give_the_groups_answers(cap, contact, mode):
+    """A lane per query -- forced, and by the rule with light and heavy queries
+    and bad ids in one batch -- against lane groups, all outputs equal."""
+    n = 4000 if mode == 2 else 131072 + 77
+    print("case: ordered lanes mode=%d cap=%d contact=%d" % (mode, cap, contact), flush=True)
+    local = F.Context(0)
+    m = [local.mesh(*TRIANGLE), local.mesh(*BOX), local.mesh(*F.icosphere(4, 0.15, 8))]
+    qm = np.random.default_rng(cap).integers(0, 3, (n, 2)).astype(np.int32)
+    qm = np.array(m, np.int32)[qm]
+    qm[::1001, 0] = 77
+    got = []
+    for v in (1, mode):
+        local.set_engine_param("ordered_lanes", v)
+        got.append(_answers(local, qm, n, cap, contact))
+    assert got[0][0] == got[1][0] != 0
+    assert all(np.array_equal(a, b) for a, b in zip(got[0][1], got[1][1]))
+    assert not got[0][1][0][::1001].any() and 0 < (got[0][1][0] > 0).mean() < 1
+    local.close()
+
+
+@pytest.mark.parametrize("n", [511, 512, 513, 32768])
+@pytest.mark.parametrize("meshes", [(TRIANGLE, TRIANGLE), (TRIANGLE, BOX)])
+def test_light_contexts(n, meshes):
+    """Contexts whose every query is light, around the sizes where the rule
+    changes, scaled matrices among them."""
+    print("case: ordered lanes, light context n=%d" % n, flush=True)
+    local = F.Context(0)
+    m = np.array([local.mesh(*x) for x in meshes], np.int32)
+    qm = np.tile(m, (n, 1))
+    tf1, tf2 = F.poses(n, 0, 1.2, 0, n)
+    tf2[::7, :9] *= 1.3
+    _same(local, qm, tf1, tf2, 1, True)
+    _same(local, qm, tf1, tf2, 5, True)
+    local.close()
