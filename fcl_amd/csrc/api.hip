@@ -825,12 +825,13 @@ int fclx_distance_batch(fclx_context* ctx, const fclx_distance_batch_args* a, vo
   hipStream_t s = static_cast<hipStream_t>(stream);
   int depth, nmesh;
   bool merged;
-  size_t nodes;
+  size_t nodes, nodes_min;
   const MeshDev* table;
   {
     std::lock_guard<std::mutex> lock(ctx->mu);
     depth = max_depth(ctx);
     nodes = max_nodes(ctx);
+    nodes_min = min_nodes(ctx);
     nmesh = static_cast<int>(ctx->meshes.size());
     table = ctx->d_table;
     merged = any_merged(ctx);
@@ -860,12 +861,15 @@ int fclx_distance_batch(fclx_context* ctx, const fclx_distance_batch_args* a, vo
   // when every bound is a lower bound of the pairs below it; merged BVs
   // need not be, and then only the reference's own order gives its answer.
   hipError_t e;
-  if (a->engine == FCLX_ENGINE_FAST && !merged)
+  L.lanes_max = kAllLanes;
+  if (a->engine == FCLX_ENGINE_FAST && !merged) {
     e = launch_distance_wave(L, 2 * depth, tu, s);
-  else if (a->engine == FCLX_ENGINE_FAST && distance_ordered_takes(nodes))
+  } else if (a->engine == FCLX_ENGINE_FAST && distance_ordered_takes(nodes)) {
+    L.lanes_max = lanes_max(ctx, distance_lanes_max(a->num_queries, nodes_min, nodes));
     e = launch_distance_ordered(L, 2 * depth, s);
-  else
+  } else {
     e = launch_distance_plain(L, 2 * depth, s);
+  }
   if (e != hipSuccess) return hip_fail(ctx, e, "distance launch");
   return FCLX_OK;
 }
@@ -1530,6 +1534,7 @@ int fclx_distance(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_
   const bool ordered = depth <= kMaxStack &&
                        distance_ordered_takes(std::max(ctx->meshes[mesh1].bvh.nodes.size(),
                                                        ctx->meshes[mesh2].bvh.nodes.size()));
+  L.lanes_max = ordered ? 0 : kAllLanes;
   HIP_TRY(ctx, ordered ? launch_distance_ordered(L, depth, s) : launch_distance_plain(L, depth, s));
   HIP_TRY(ctx, hipStreamSynchronize(s));
   if (!ordered) {  // the one-lane kernel can outgrow its stack

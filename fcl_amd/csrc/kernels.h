@@ -83,6 +83,7 @@ struct DistanceLaunch {
   long long* bv_tests;
   long long* leaf_tests;
   int32_t* status;
+  long long lanes_max;         // as in CollideLaunch (the plain kernel's: kAllLanes)
 };
 
 // Primitive-shape pairs (records in the fclx_shape layout of fclx.h)
@@ -218,6 +219,7 @@ hipError_t launch_distance_plain(const DistanceLaunch& L, int stack_need, hipStr
 // distance() in the reference's order, a wavefront per query
 // (kernels_clearance.hip); its entries hold node indices below 2^26
 bool distance_ordered_takes(size_t max_nodes);
+long long distance_lanes_max(int num_queries, size_t nodes_min, size_t nodes_max);
 hipError_t launch_distance_ordered(const DistanceLaunch& L, int stack_need, hipStream_t s);
 // FAST engine: wavefront-wide search with the reference's visit order kept
 // as path keys (engine_dist.hip); BVTTs deeper than 62 levels go to the

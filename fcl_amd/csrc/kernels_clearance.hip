@@ -88,6 +88,8 @@ __device__ __forceinline__ int first_of(unsigned long long m) {
   return m != 0 ? __ffsll(static_cast<long long>(m)) - 1 : kWave;
 }
 
+// kSome: queries of L.lanes_max node pairs at most are left to a lane each.
+template <bool kSome>
 __global__ void __launch_bounds__(kWave, 1) distance_ordered(DistanceLaunch L, int margin) {
   __shared__ List S;
   const int q = blockIdx.x;
@@ -109,6 +111,7 @@ __global__ void __launch_bounds__(kWave, 1) distance_ordered(DistanceLaunch L, i
   }
   const MeshDev& m1 = L.meshes[i1];
   const MeshDev& m2 = L.meshes[i2];
+  if (kSome && node_pairs(m1, m2) <= L.lanes_max) return;
   const double* tf1 = L.tf1 + 12 * static_cast<size_t>(q);
   M3 R;
   V3 T;
@@ -344,14 +347,37 @@ __global__ void __launch_bounds__(kWave, 1) distance_ordered(DistanceLaunch L, i
 
 bool distance_ordered_takes(size_t max_nodes) { return max_nodes <= (size_t(1) << kIdBits); }
 
+// Where a lane per query is the faster form (for the queries whose chains a
+// batch is large enough to hide).  Lanes / wavefronts, measured: two triangles,
+// 2,000 queries 51 / 52 us and 1,000,000 0.32 / 9.2 ms; a triangle and a box
+// of 12, 32,768 queries 0.56 / 0.54; two boxes 65,536 3.9 / 3.5 and 131,072
+// 4.5 / 6.9; 2 x 20 triangles 65,536 5.4 / 6.1; 2 x 80, 131,072 30 / 39; 320 and
+// 80, 250,000 104 / 117; 2 x 320, 250,000 194 / 189 and 1,000,000 676 / 749; 2 x
+// 2,420, 250,000 1,518 / 1,432 ms.
+long long distance_lanes_max(int num_queries, size_t nodes_min, size_t nodes_max) {
+  long long limit = 0;
+  if (num_queries >= 2048) limit = 1;
+  if (num_queries >= 36864) limit = 64;
+  if (num_queries >= 65536) limit = 2048;
+  if (num_queries >= 98304) limit = 32768;
+  if (num_queries >= 196608) limit = 131072;
+  if (num_queries >= 600000) limit = 524288;
+  return lanes_within(limit, nodes_min, nodes_max);
+}
+
 hipError_t launch_distance_ordered(const DistanceLaunch& L, int stack_need, hipStream_t s) {
+  if (L.lanes_max > 0) {
+    const hipError_t e = launch_distance_plain(L, stack_need, s);
+    if (e != hipSuccess || L.lanes_max == kAllLanes) return e;
+  }
+  auto kernel = L.lanes_max > 0 ? distance_ordered<true> : distance_ordered<false>;
   // HIP refuses a launch of 2^32 threads: larger batches in parts (a loop in
   // the kernel took 2 % of a single call)
   constexpr int kPart = 1 << 25;
   DistanceLaunch P = L;
   for (int left = L.num_queries; left > 0; left -= kPart) {
     P.num_queries = left < kPart ? left : kPart;
-    distance_ordered<<<static_cast<unsigned>(P.num_queries), kWave, 0, s>>>(P, stack_need + 2);
+    kernel<<<static_cast<unsigned>(P.num_queries), kWave, 0, s>>>(P, stack_need + 2);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     P.query_meshes += 2 * static_cast<size_t>(kPart);

@@ -269,6 +269,7 @@ __global__ void __launch_bounds__(256) distance_plain_kernel(DistanceLaunch L) {
   }
   const MeshDev m1 = L.meshes[i1];
   const MeshDev m2 = L.meshes[i2];
+  if (node_pairs(m1, m2) > L.lanes_max) return;
   const double* tf1 = L.tf1 + 12 * static_cast<size_t>(q);
   const double* tf2 = L.tf2 + 12 * static_cast<size_t>(q);
   M3 R;

@@ -75,3 +75,35 @@ def test_merged_bvs_follow_the_reference_order(ctx):
     got = _batch(local, m, tf1, tf2, F.ENGINE_FAST)
     assert all(np.array_equal(a, b) for a, b in zip(got, want))
     local.close()
+
+
+@pytest.mark.parametrize("mode,n", [(2, 300), (0, 2047), (0, 2048), (0, 65536 + 5)])
+def test_lanes_give_the_wavefronts_answers(mode, n):
+    """Merged BVs with a lane per query -- forced, and by the rule with light
+    and heavy queries and bad ids in one batch -- against wavefronts."""
+    print("case: clearance lanes mode=%d n=%d" % (mode, n), flush=True)
+    local = F.Context(0)
+    tri = np.array([[0.9, 0, 0], [-0.4, 0.8, 0], [-0.4, -0.8, 0.1]]), np.array([[0, 1, 2]])
+    heavy = F.icosphere(3, 0.15, 8)
+    m = np.array([local.mesh(*x, F.RSS) for x in (tri, F.icosphere(1, 0.1, 9), heavy)], np.int32)
+    local.mesh_refit(int(m[1]), torch.from_numpy(F.icosphere(1, 0.1, 9)[0] * 1.05).to(DEV),
+                     bottomup=True)
+    qm = m[np.random.default_rng(n).integers(0, 3, (n, 2))]
+    qm[5::500, 1] = -1
+    tf1, tf2 = F.poses(n, 1, 1.9, 4.0, 0xD17)
+    out = []
+    for v in (1, mode):
+        local.set_engine_param("ordered_lanes", v)
+        d = torch.full((n,), -1, dtype=torch.float64, device=DEV)
+        p = torch.zeros((n, 6), dtype=torch.float64, device=DEV)
+        i = torch.full((n, 2), -7, dtype=torch.int32, device=DEV)
+        st = [torch.full((n,), -1, dtype=torch.int64, device=DEV) for _ in range(2)]
+        s = torch.cuda.current_stream().cuda_stream
+        local.distance_batch_async(_t(qm, torch.int32), _t(tf1, torch.float64),
+                                   _t(tf2, torch.float64), d, p, i, engine=F.ENGINE_FAST,
+                                   bv_tests=st[0], leaf_tests=st[1], stream=s)
+        assert local.sync_status(s) != 0
+        good = torch.from_numpy((qm >= 0).all(1)).to(DEV)
+        out.append([d, i] + st + [p[good]])
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+    local.close()
