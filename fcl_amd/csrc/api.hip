@@ -115,6 +115,8 @@ struct fclx_context {
   std::atomic<int> serve_fail_launches{0};  // failure injection for the serving loop
   std::atomic<uint32_t> ordered_carry_max{1u << 31};
   std::atomic<int> ordered_lanes{0};
+  std::atomic<int> meshshape_list_depth{kMsListDepth};
+  std::atomic<size_t> meshshape_epa_queue{kMsEpaQueue};
 };
 
 namespace {
@@ -885,11 +887,14 @@ int fclx_mesh_shape_collide_batch(fclx_context* ctx, const fclx_mesh_shape_colli
        (!a->contact_pos || !a->contact_normal || !a->contact_depth)))
     return fail(ctx, FCLX_ERR_INVALID_ARGUMENT, "invalid mesh-shape batch arguments");
   MeshShapeLaunch L{};
+  size_t nodes, nodes_min;
   {
     std::lock_guard<std::mutex> lock(ctx->mu);
     L.meshes = ctx->d_table;
     L.num_meshes = static_cast<int32_t>(ctx->meshes.size());
     L.max_depth = max_depth(ctx);
+    nodes = max_nodes(ctx);
+    nodes_min = min_nodes(ctx);
   }
   (void)hipSetDevice(ctx->device);
   L.num_queries = a->num_queries;
@@ -912,6 +917,10 @@ int fclx_mesh_shape_collide_batch(fclx_context* ctx, const fclx_mesh_shape_colli
   L.stats = reinterpret_cast<long long*>(a->stats);
   L.status = ctx->d_status;
   L.carry_max = ctx->ordered_carry_max.load();
+  L.lanes_max = lanes_max(ctx, mesh_shape_lanes_max(a->num_queries, a->num_max_contacts, nodes_min,
+                                                    nodes));
+  L.list_depth = ctx->meshshape_list_depth.load();
+  L.epa_queue = ctx->meshshape_epa_queue.load();
   int waves;
   {
     std::lock_guard<std::mutex> lock(ctx->ws_mu);
@@ -1086,6 +1095,8 @@ int fclx_get_engine_param(fclx_context* ctx, const char* name, double* value) {
   else if (n == "meshshape_leaf_share") *value = t.meshshape_leaf_share;
   else if (n == "ordered_carry_max") *value = ctx->ordered_carry_max.load();
   else if (n == "ordered_lanes") *value = ctx->ordered_lanes.load();
+  else if (n == "meshshape_list_depth") *value = ctx->meshshape_list_depth.load();
+  else if (n == "meshshape_epa_queue") *value = static_cast<double>(ctx->meshshape_epa_queue.load());
   else if (n == "dist_width") *value = t.dist.width;
   else if (n == "dist_leaf_batch") *value = t.dist.leaf_batch;
   else if (n == "dist_fp32_cull") *value = t.dist.fp32_cull;
@@ -1146,6 +1157,10 @@ int fclx_set_engine_param(fclx_context* ctx, const char* name, double value) {
     ctx->ordered_carry_max.store(static_cast<uint32_t>(value));
   } else if (n == "ordered_lanes" && (value == 0 || value == 1 || value == 2)) {
     ctx->ordered_lanes.store(static_cast<int>(value));
+  } else if (n == "meshshape_list_depth" && in(0, kMsListDepth)) {
+    ctx->meshshape_list_depth.store(static_cast<int>(value));
+  } else if (n == "meshshape_epa_queue" && in(0, static_cast<double>(kMsEpaQueue))) {
+    ctx->meshshape_epa_queue.store(static_cast<size_t>(value));
   } else if (n == "dist_width" && in(1, 64)) {
     t.dist.width = static_cast<int>(value);
   } else if (n == "dist_leaf_batch" && in(1, 64)) {

@@ -108,6 +108,8 @@ struct ShapeLaunch {
 };
 
 // Mesh (BVHModel<OBBRSS>) against a primitive shape.
+constexpr int kMsListDepth = 440;  // deepest mesh whose descent a list in LDS holds beside a step
+constexpr size_t kMsEpaQueue = size_t(4) << 30;  // bytes of queued EPA work at most
 struct MeshShapeLaunch {
   const MeshDev* meshes;        // device table indexed by mesh id
   int32_t num_meshes;
@@ -133,11 +135,16 @@ struct MeshShapeLaunch {
   int32_t leaf_share;           // percent of a wavefront's lanes with a leaf that starts a
                                 // leaf round (1..100; 0: 100)
   uint32_t carry_max;           // most BV tests that a query's list carries
+  int32_t list_depth;           // at most kMsListDepth (lower in tests)
+  size_t epa_queue;             // at most kMsEpaQueue (lower in tests)
+  long long lanes_max;          // queries on meshes of at most this many nodes run on a lane
+                                // each: none, some of the batch, or kAllLanes
   int32_t max_depth;            // deepest mesh of the context (levels)
 };
 // waves: register budget, 1..3 waves per SIMD
 hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& L, int waves, hipStream_t s);
 size_t mesh_shape_epa_lane_bytes();
+long long mesh_shape_lanes_max(int num_queries, int cap, size_t nodes_min, size_t nodes_max);
 
 hipError_t launch_collide_plain(const CollideLaunch& L, int stack_need, hipStream_t s);
 // a query per lane with FP32 culls, for the queries of L.lanes_max node pairs

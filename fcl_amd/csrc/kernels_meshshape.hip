@@ -38,12 +38,14 @@ namespace {
 
 constexpr int kBlk = 256;
 constexpr int kMsListCap = 512;    // entries of a query's list in LDS
-constexpr int kMsListDepth = 440;  // deepest mesh whose descent it holds beside a step
-// deeper meshes (up to kMsDeepMax levels) keep a stack in device memory
+static_assert(kMsListDepth + 2 + 64 <= kMsListCap, "a tree path and a step");
+// Lanes keep their pending right children in LDS up to this depth; in contexts
+// with meshes deeper than MeshShapeLaunch::list_depth (up to kMsDeepMax levels) in device
+// memory.
+constexpr int kMsLaneStack = 64;
 constexpr int kMsDeepMax = 4096;
 constexpr int kMsDeepBlocksPerCu = 2;
 constexpr int kEpaBlocksPerCu = 2;
-constexpr size_t kEpaQueueBudget = size_t(4) << 30;  // bytes of queued EPA seeds at most
 
 // A hit whose contact EPA supplies: the query, the triangle and the record
 // slot the contact goes to.
@@ -354,6 +356,58 @@ __device__ __forceinline__ bool load_query(const MeshShapeLaunch& L, int q, shp:
   return false;
 }
 
+// For lanes: the queries grouped by shape kind, so that a wavefront's lanes run
+// the same leaf test (their order does not change any query's answer).  Keys:
+// the five kinds, 5 for a query whose mesh or shape id is out of range, and
+// 6, last, for those of more than L.lanes_max nodes, which run on wavefronts.
+// ctr[0..6]: counts, ctr[8..14]: placement cursors.
+constexpr int kKinds = 7;
+
+__device__ __forceinline__ int kind_of(const MeshShapeLaunch& L, int q) {
+  const int mi = L.query_meshes[q], si = L.query_shapes[q];
+  if (mi < 0 || mi >= L.num_meshes || si < 0 || si >= L.num_shapes) return 5;
+  if (L.lanes_max != kAllLanes && L.meshes[mi].num_bvs > L.lanes_max) return 6;
+  const int t = L.shapes[si].type;
+  return t >= 0 && t < 5 ? t : 5;
+}
+
+__global__ void ms_zero(int32_t* ctr) {
+  if (threadIdx.x < 16) ctr[threadIdx.x] = 0;
+}
+
+__global__ void __launch_bounds__(kBlk) ms_count(MeshShapeLaunch L, int32_t* ctr) {
+  __shared__ int cnt[kKinds];
+  if (threadIdx.x < kKinds) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int i = blockIdx.x * kBlk + threadIdx.x;
+  if (i < L.num_queries) atomicAdd(&cnt[kind_of(L, i)], 1);
+  __syncthreads();
+  if (threadIdx.x < kKinds && cnt[threadIdx.x]) atomicAdd(&ctr[threadIdx.x], cnt[threadIdx.x]);
+}
+
+__global__ void __launch_bounds__(kBlk) ms_place(MeshShapeLaunch L, int32_t* ctr,
+                                                 int32_t* order) {
+  __shared__ int cnt[kKinds];
+  __shared__ int base[kKinds];
+  if (threadIdx.x < kKinds) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  const int i = blockIdx.x * kBlk + threadIdx.x;
+  int key = 0, off = 0;
+  if (i < L.num_queries) {
+    key = kind_of(L, i);
+    off = atomicAdd(&cnt[key], 1);
+  }
+  __syncthreads();
+  if (threadIdx.x < kKinds) {
+    int start = 0;
+    for (int k = 0; k < static_cast<int>(threadIdx.x); ++k) start += ctr[k];
+    base[threadIdx.x] =
+        start + (cnt[threadIdx.x] ? atomicAdd(&ctr[8 + threadIdx.x], cnt[threadIdx.x]) : 0);
+  }
+  __syncthreads();
+  if (i < L.num_queries) order[base[key] + off] = i;
+}
+
 // The leaf test of one (shape, triangle) pair, kept out of line so that the
 // descent loop's registers are not sized for GJK and EPA.
 template <bool kContact>
@@ -408,6 +462,7 @@ static_assert(sizeof(MsQuery) == 128, "one line per query");
 __global__ void __launch_bounds__(kBlk) meshshape_setup(MeshShapeLaunch L, MsQuery* out) {
   const int q = blockIdx.x * kBlk + threadIdx.x;
   if (q >= L.num_queries) return;
+  if (L.lanes_max > 0 && kind_of(L, q) != 6) return;  // a lane's
   MsQuery r;
   shp::Shape s;
   r.valid = load_query(L, q, s, L.max_depth) ? 1 : 0;
@@ -445,8 +500,7 @@ struct MsWave {
 };
 
 // The leaf test's answer alone: a sphere by the closed form, the other
-// shapes by GJK.  Out of line, so that the traversal's registers are not
-// sized for it.
+// shapes by GJK.
 __device__ __forceinline__ bool leaf_inside(const MsWave& w, const double* tv, double tol) {
   if (w.s.type == shp::kSphere) {
     D3 P[3];
@@ -483,7 +537,7 @@ __device__ __forceinline__ bool leaf_inside(const MsWave& w, const double* tv, d
 // query, as before, took 330-460 ms for this batch, the time of its longest
 // query; 200,000 links that nearly all collide at once 8.3 ms, now 7.3.
 // Quarter wavefronts are faster for the latter (4.2 ms) and slower for the
-// former (28 ms).
+// former (28 ms).  Large batches on small meshes run on lanes (below).
 template <bool kStats, bool kContact>
 __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery* queries, size_t q,
                                         int margin, int leaf_min, MsEpaSeed* seeds,
@@ -635,62 +689,84 @@ template <bool kStats, bool kContact, int kWaves>
 __global__ void __launch_bounds__(64, kWaves) meshshape_ordered(MeshShapeLaunch L,
                                                                 const MsQuery* queries, int margin,
                                                                 int leaf_min, MsEpaSeed* seeds,
-                                                                unsigned long long* nseed) {
+                                                                unsigned long long* nseed,
+                                                                const int32_t* order,
+                                                                const int32_t* ctr) {
   __shared__ OrderedList<kMsListCap, kStats> S;
   __shared__ MsWave w;
-  for (size_t q = blockIdx.x; q < static_cast<size_t>(L.num_queries); q += gridDim.x)
-    descend<kStats, kContact>(L, queries, q, margin, leaf_min, seeds, nseed, S, w);
+  // all queries, or the order's last part
+  const size_t end = L.num_queries, first = order ? end - static_cast<size_t>(ctr[6]) : 0;
+  for (size_t k = first + blockIdx.x; k < end; k += gridDim.x)
+    descend<kStats, kContact>(L, queries, order ? static_cast<size_t>(order[k]) : k, margin,
+                              leaf_min, seeds, nseed, S, w);
 }
 
-// Lanes of a wavefront step together: a lane whose descent reached a leaf
-// that passed its BV test waits there, the others keep descending, and the
-// waiting lanes test their leaves together once they are a set share of the
-// live lanes (or nobody can descend).  The costly leaf test (GJK) then
-// runs once for many lanes instead of once per descent step.  Each lane's
-// own order of tests is the reference's, so counts, triangles and test
+// A query per lane.  Lanes of a wavefront step together: a lane whose descent
+// reached a leaf that passed its BV test waits there, the others keep
+// descending, and the waiting lanes test their leaves together once they are a
+// set share of the live lanes (or nobody can descend).  The costly leaf test
+// (GJK) then runs once for many lanes instead of once per descent step.  Each
+// lane's own order of tests is the reference's, so counts, triangles and test
 // statistics are unchanged.
 //
-// For what the lists in LDS do not hold: contexts with a mesh deeper than
-// kMsListDepth, and contact batches whose EPA queue would exceed its budget
-// (EPA then runs in the descending lane).  The pending right children live
-// in device memory (one column of L.max_depth entries per lane,
-// lane-interleaved).
-template <bool kContact>
-__global__ void __launch_bounds__(kBlk, 1) meshshape_deep(MeshShapeLaunch L, shp::EpaLane* lanes,
-                                                          shp::EpaWave* waves,
-                                                          int* deep_stack) {
+// For the light queries of large batches (order: those grouped by kind, ctr:
+// the groups' counts; the rule is at mesh_shape_lanes_max), whose hits are queued
+// for EPA; and for what the lists in LDS do not hold: contexts with a mesh
+// deeper than L.list_depth, and contact batches whose EPA queue would exceed
+// its budget (EPA then runs in the descending lane).
+//
+// kDeep: the pending right children live in device memory (deep_stack, one
+// column of L.max_depth entries per lane, lane-interleaved) instead of LDS.
+template <bool kContact, bool kDeep, bool kQueue>
+__global__ void __launch_bounds__(kBlk, kDeep ? 1 : 2) meshshape_lanes(
+    MeshShapeLaunch L, const int32_t* order, const int32_t* ctr, shp::EpaLane* lanes,
+    shp::EpaWave* waves, int* deep_stack, MsEpaSeed* seeds, unsigned long long* nseed) {
+  constexpr bool kEpaHere = kContact && !kQueue;
   const size_t gid = static_cast<size_t>(blockIdx.x) * kBlk + threadIdx.x;
   const size_t stride = static_cast<size_t>(gridDim.x) * kBlk;
+  const size_t end = static_cast<size_t>(L.num_queries) - (order ? static_cast<size_t>(ctr[6]) : 0);
   // the horizon walk's stack in LDS, one column per thread
-  __shared__ int16_t xs_lds[kContact ? shp::kNfEpa : 1][kBlk];
+  __shared__ int16_t xs_lds[kEpaHere ? shp::kNfEpa : 1][kBlk];
   shp::Epa E;
-  if constexpr (kContact) {
+  if constexpr (kEpaHere) {
     E.M = lanes + gid;
     E.S = waves + gid / 64;
     E.lane = threadIdx.x & 63;
     E.xs = &xs_lds[0][threadIdx.x];
     E.xs_stride = kBlk;
   }
-  size_t q = gid;
+  size_t qq = gid;  // position in the order
+  size_t q = 0;     // the query at that position
   shp::Shape s;
   shp::Xf T1, T2;
   double sa[9], sto[3], sext[3];
   const ObbNode64* nodes = nullptr;
   const double* tris = nullptr;
+  // pending right children in LDS, one column per lane (lane-interleaved:
+  // conflict-free whatever depth each lane is at)
+  __shared__ int stk[kDeep ? 1 : kMsLaneStack][kBlk];
+  const int column = threadIdx.x;
   int sp = 0, b = 0, count = 0, pend = -1;
   long long nbv = 0, nleaf = 0;
   bool live = false;  // a query in progress
   auto push = [&](int v) {
-    deep_stack[static_cast<size_t>(sp) * stride + gid] = v;
+    if constexpr (kDeep)
+      deep_stack[static_cast<size_t>(sp) * stride + gid] = v;
+    else
+      stk[sp][column] = v;
     ++sp;
   };
   auto pop = [&]() -> int {
     --sp;
-    return deep_stack[static_cast<size_t>(sp) * stride + gid];
+    if constexpr (kDeep)
+      return deep_stack[static_cast<size_t>(sp) * stride + gid];
+    else
+      return stk[sp][column];
   };
   // take queries until one is usable (the others are answered at once)
   auto start = [&]() {
-    while (q < static_cast<size_t>(L.num_queries)) {
+    while (qq < end) {
+      q = order ? static_cast<size_t>(order[qq]) : qq;
       if (load_query(L, static_cast<int>(q), s, L.max_depth)) {
         const MeshDev& M = L.meshes[L.query_meshes[q]];
         nodes = M.obb64;
@@ -713,7 +789,7 @@ __global__ void __launch_bounds__(kBlk, 1) meshshape_deep(MeshShapeLaunch L, shp
         L.stats[2 * q + 1] = 0;
       }
       atomicOr(L.status, kStatusBadQuery);
-      q += stride;
+      qq += stride;
     }
     live = false;
   };
@@ -723,7 +799,7 @@ __global__ void __launch_bounds__(kBlk, 1) meshshape_deep(MeshShapeLaunch L, shp
       L.stats[2 * q] = nbv;
       L.stats[2 * q + 1] = nleaf;
     }
-    q += stride;
+    qq += stride;
     start();
   };
   auto next = [&]() {  // the next node of the descent, or the query's end
@@ -745,18 +821,35 @@ __global__ void __launch_bounds__(kBlk, 1) meshshape_deep(MeshShapeLaunch L, shp
       ++nleaf;
       shp::Contact c;
       const bool hit =
-          leaf_test<kContact>(s, T1, T2, tris + static_cast<size_t>(prim) * kTriVertsStride, L.tol,
+          leaf_test<kEpaHere>(s, T1, T2, tris + static_cast<size_t>(prim) * kTriVertsStride, L.tol,
                               E, c);
+      const bool queued = kQueue && s.type != shp::kSphere;
+      if constexpr (kQueue) {
+        // the hits of this leaf round for EPA: one reservation for the wavefront
+        const unsigned long long em = __ballot(hit && queued);
+        if (em != 0) {
+          const int leader = __ffsll(static_cast<long long>(em)) - 1;
+          unsigned long long at = 0;
+          if (static_cast<int>(threadIdx.x & 63) == leader)
+            at = atomicAdd(nseed, static_cast<unsigned long long>(__popcll(em)));
+          at = __shfl(at, leader);
+          if (hit && queued)
+            seeds[at + __popcll(em & ((1ULL << (threadIdx.x & 63)) - 1ULL))] = MsEpaSeed{
+                static_cast<int32_t>(q), prim, static_cast<long long>(q * L.cap + count)};
+        }
+      }
       if (hit) {
         const size_t k = q * L.cap + count;
         if (L.prims) L.prims[k] = prim;
         if constexpr (kContact) {
+          if (!queued) {
 #pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            L.contact_pos[3 * k + j] = c.pos.v[j];
-            L.contact_normal[3 * k + j] = c.normal.v[j];
+            for (int j = 0; j < 3; ++j) {
+              L.contact_pos[3 * k + j] = c.pos.v[j];
+              L.contact_normal[3 * k + j] = c.normal.v[j];
+            }
+            L.contact_depth[k] = c.depth;
           }
-          L.contact_depth[k] = c.depth;
         }
         if (++count >= L.cap) {
           finish();
@@ -882,20 +975,27 @@ namespace {
 
 template <int kWaves>
 void launch_descent(const MeshShapeLaunch& L, const MsQuery* queries, MsEpaSeed* seeds,
-                    unsigned long long* nseed, hipStream_t s) {
+                    unsigned long long* nseed, const int32_t* order, const int32_t* ctr,
+                    hipStream_t s) {
   auto kernel = L.contact ? (L.stats ? meshshape_ordered<true, true, kWaves>
                                      : meshshape_ordered<false, true, kWaves>)
                           : (L.stats ? meshshape_ordered<true, false, kWaves>
                                      : meshshape_ordered<false, false, kWaves>);
   const int leaf_min = L.leaf_share > 0 ? std::max(1, 64 * L.leaf_share / 100) : 64;
   kernel<<<group_blocks(L.num_queries), 64, 0, s>>>(L, queries, L.max_depth + 2, leaf_min, seeds,
-                                                    nseed);
+                                                    nseed, order, ctr);
+}
+
+// Leaf rounds of the lanes, measured: at half the live lanes for booleans, three
+// quarters with contact geometry.
+int lane_leaf_share(const MeshShapeLaunch& L) {
+  return L.leaf_share > 0 ? L.leaf_share : (L.contact ? 75 : 50);
 }
 
 // Stream-ordered scratch of one batch, freed (in stream order) at its end.
 struct StreamScratch {
   hipStream_t s;
-  void* held[4] = {};
+  void* held[8] = {};
   int n = 0;
   explicit StreamScratch(hipStream_t stream) : s(stream) {}
   ~StreamScratch() {
@@ -920,28 +1020,58 @@ struct StreamScratch {
   } while (0)
 
 hipError_t launch_deep(MeshShapeLaunch L, int cus, hipStream_t s) {
-  // measured: leaf rounds at half the live lanes for booleans, three
-  // quarters with contact geometry
-  if (L.leaf_share <= 0) L.leaf_share = L.contact ? 75 : 50;
+  L.leaf_share = lane_leaf_share(L);
   long long grid = (static_cast<long long>(L.num_queries) + kBlk - 1) / kBlk;
   grid = std::min<long long>(grid, static_cast<long long>(cus) * kMsDeepBlocksPerCu);
   const size_t lanes = static_cast<size_t>(grid) * kBlk;
   StreamScratch mem(s);
   int* stack = nullptr;
   MS_TRY(mem.get(&stack, lanes * L.max_depth));
-  if (!L.contact) {
-    meshshape_deep<false><<<static_cast<unsigned>(grid), kBlk, 0, s>>>(L, nullptr, nullptr, stack);
-    return hipGetLastError();
-  }
   shp::EpaLane* el = nullptr;
   shp::EpaWave* ew = nullptr;
-  MS_TRY(mem.get(&el, lanes));
-  MS_TRY(mem.get(&ew, lanes / 64));
-  meshshape_deep<true><<<static_cast<unsigned>(grid), kBlk, 0, s>>>(L, el, ew, stack);
+  if (L.contact) {
+    MS_TRY(mem.get(&el, lanes));
+    MS_TRY(mem.get(&ew, lanes / 64));
+  }
+  auto kernel = L.contact ? meshshape_lanes<true, true, false> : meshshape_lanes<false, true, false>;
+  kernel<<<static_cast<unsigned>(grid), kBlk, 0, s>>>(L, nullptr, nullptr, el, ew, stack, nullptr,
+                                                      nullptr);
+  return hipGetLastError();
+}
+
+// The queries of L.lanes_max nodes at most (all with kAllLanes) on a lane each.
+// order, ctr: filled for launch_descent to take the others from.
+hipError_t launch_lanes(MeshShapeLaunch L, MsEpaSeed* seeds, unsigned long long* nseed,
+                        int32_t* order, int32_t* ctr, hipStream_t s) {
+  L.leaf_share = lane_leaf_share(L);
+  const unsigned grid = static_cast<unsigned>((L.num_queries + kBlk - 1) / kBlk);
+  ms_zero<<<1, 64, 0, s>>>(ctr);
+  ms_count<<<grid, kBlk, 0, s>>>(L, ctr);
+  ms_place<<<grid, kBlk, 0, s>>>(L, ctr, order);
+  auto kernel = L.contact ? meshshape_lanes<true, false, true> : meshshape_lanes<false, false, false>;
+  kernel<<<grid, kBlk, 0, s>>>(L, order, ctr, nullptr, nullptr, nullptr, seeds, nseed);
   return hipGetLastError();
 }
 
 }  // namespace
+
+// Where a lane per query is the faster form: on small meshes, in batches large
+// enough to hide the lanes' waiting for each other's leaf rounds, which grows
+// with the mesh (and with the contacts asked for).  Lanes / wavefronts, to the
+// first hit: a triangle, 32,768 queries 249 / 314 us and 1,000,000 1.0 / 5.8 ms;
+// 12 triangles 65,536 1.5 / 0.8, 131,072 1.4 / 1.4 and 1,000,000 4.6 / 10.3; 80
+// triangles 131,072 2.74 / 2.68 and 250,000 3.6 / 5.0; 180 triangles 250,000 5.9 /
+// 5.8; 320 triangles 500,000 12.2 / 12.4 and 1,000,000 20 / 25; 800 triangles
+// 3,000,000 87 / 79.  To 4 hits: 80 triangles 131,072 3.7 / 2.7 and 250,000 4.8 /
+// 5.0; 180 triangles 500,000 10.4 / 11.4; 320 triangles 1,000,000 26 / 25 and
+// 3,000,000 67 / 71.
+long long mesh_shape_lanes_max(int num_queries, int cap, size_t nodes_min, size_t nodes_max) {
+  long long limit = num_queries >= 24576 ? 1 : 0;
+  const long long over = (num_queries - 90112LL) / (cap > 1 ? 3 : 1);
+  while (limit < 1023 && (limit + 1) * (limit + 1) <= over) ++limit;
+  if (static_cast<long long>(nodes_min) > limit) return 0;
+  return static_cast<long long>(nodes_max) <= limit ? kAllLanes : limit;
+}
 
 hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& in, int waves, hipStream_t s) {
   if (in.num_queries <= 0) return hipSuccess;
@@ -951,22 +1081,33 @@ hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& in, int waves, hipSt
   MS_TRY(hipGetDevice(&dev));
   MS_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const size_t nslots = static_cast<size_t>(L.num_queries) * static_cast<size_t>(L.cap);
-  if (L.max_depth > kMsListDepth || (L.contact && nslots > kEpaQueueBudget / sizeof(MsEpaSeed)))
+  if (L.max_depth > L.list_depth || (L.contact && nslots > L.epa_queue / sizeof(MsEpaSeed)))
     return launch_deep(L, cus, s);
+  if (L.max_depth > kMsLaneStack) L.lanes_max = 0;
   StreamScratch mem(s);
   MsQuery* queries = nullptr;
   MsEpaSeed* seeds = nullptr;
   unsigned long long* ctr = nullptr;  // [0] seeds queued, [1] seeds handed out
-  MS_TRY(mem.get(&queries, static_cast<size_t>(L.num_queries)));
+  int32_t* order = nullptr;
+  int32_t* kinds = nullptr;
   if (L.contact) {
     MS_TRY(mem.get(&seeds, nslots));
     MS_TRY(mem.get(&ctr, 2));
     ms_zero_u64<<<1, 64, 0, s>>>(ctr);
   }
-  meshshape_setup<<<static_cast<unsigned>((L.num_queries + kBlk - 1) / kBlk), kBlk, 0, s>>>(
-      L, queries);
-  auto descent = waves == 1 ? launch_descent<1> : (waves == 3 ? launch_descent<3> : launch_descent<2>);
-  descent(L, queries, seeds, ctr, s);
+  if (L.lanes_max > 0) {
+    MS_TRY(mem.get(&order, static_cast<size_t>(L.num_queries)));
+    MS_TRY(mem.get(&kinds, 16));
+    MS_TRY(launch_lanes(L, seeds, ctr, order, kinds, s));
+  }
+  if (L.lanes_max != kAllLanes) {
+    MS_TRY(mem.get(&queries, static_cast<size_t>(L.num_queries)));
+    meshshape_setup<<<static_cast<unsigned>((L.num_queries + kBlk - 1) / kBlk), kBlk, 0, s>>>(
+        L, queries);
+    auto descent =
+        waves == 1 ? launch_descent<1> : (waves == 3 ? launch_descent<3> : launch_descent<2>);
+    descent(L, queries, seeds, ctr, order, kinds, s);
+  }
   MS_TRY(hipGetLastError());
   if (!L.contact) return hipSuccess;
   const long long egrid = static_cast<long long>(cus) * kEpaBlocksPerCu;

@@ -267,9 +267,9 @@ int fclx_collide_batch_noalloc(fclx_context* ctx, const fclx_collide_batch_args*
  * query naming a missing mesh or shape, an RSS mesh, a mesh deeper than 4096
  * levels or a convex with fewer than 4 vertices gets count 0 and makes
  * fclx_sync return FCLX_ERR_INVALID_ARGUMENT.  A call takes
- * stream-ordered device memory, freed when the batch ends: 128 bytes per
- * query, with enable_contact also for EPA (16 bytes per slot and about 12 KB
- * per resident lane), and, while the context holds a mesh deeper than 440
+ * stream-ordered device memory, freed when the batch ends: up to 132 bytes
+ * per query, with enable_contact also for EPA (16 bytes per slot and about 12
+ * KB per resident lane), and, while the context holds a mesh deeper than 440
  * levels, for descent stacks (4 bytes per level per resident lane). */
 typedef struct {
   int32_t num_queries;
@@ -399,7 +399,14 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *   "meshshape_leaf_share" 0..100  percent of a wavefront's lanes with a leaf
  *                               to test that starts their leaf tests
  *                               (default 0: 100, or when nothing else is
- *                               left to test)
+ *                               left to test; with a lane per query 50 of
+ *                               the live ones, 75 with contact geometry)
+ *   "meshshape_list_depth" 0..440  deepest mesh (levels) of a context whose
+ *                               mesh-shape batches descend in LDS (default
+ *                               440: deeper ones use device memory)
+ *   "meshshape_epa_queue" 0..2^32  bytes of queued EPA work of a mesh-shape
+ *                               batch (16 per slot; default 2^32: above it
+ *                               EPA runs in the descending lanes)
  *   "ordered_carry_max" 1..2^31 test counts that the traversals in the
  *                               reference's order hold ahead of their turn
  *                               before they go one node at a time (default

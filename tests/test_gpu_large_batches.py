@@ -38,10 +38,13 @@ def _repeats(got, want):
     return bool((whole == w).all()) and bool((got[n - n % PERIOD:] == w[:n % PERIOD]).all())
 
 
-@pytest.mark.parametrize("n,cap,contact", [(BLOCKS + 77, 2, True), (4 * BLOCKS + 77, 1, False),
-                                           (PAST, 2, False), (PAST, 2, True)])
-def test_collide(ctx, poses, n, cap, contact):
-    print("case: %d collide queries, contact=%d" % (n, contact), flush=True)
+@pytest.mark.parametrize("n,cap,contact,lanes",
+                         [(BLOCKS + 77, 2, True, 1), (4 * BLOCKS + 77, 1, False, 1),
+                          (PAST, 2, False, 1), (PAST, 2, True, 1), (PAST, 1, False, 2)])
+def test_collide(poses, n, cap, contact, lanes):
+    print("case: %d collide queries, contact=%d lanes=%d" % (n, contact, lanes), flush=True)
+    ctx = F.Context(0)
+    ctx.set_engine_param("ordered_lanes", lanes)
     m = [ctx.mesh(*F.icosphere(2, 0.15, k)) for k in (1, 2)]
     want = collide_gpu(ctx, np.tile(np.array(m, np.int32), (PERIOD, 1)), *poses, cap)[1]
     if contact:
@@ -61,12 +64,14 @@ def test_collide(ctx, poses, n, cap, contact):
                             engine=F.ENGINE_FAST, contact=geo, stream=s)
     ctx.sync_status(s)  # (more contacts than rows)
     assert _repeats(counts, want) and int(num.item()) == int(counts.long().sum())
+    ctx.close()
 
 
 @pytest.mark.parametrize("n", [PAST])
 def test_distance_over_merged_bvs(n):
     print("case: %d distance queries" % n, flush=True)
     local = F.Context(0)
+    local.set_engine_param("ordered_lanes", 1)
     V, T = F.icosphere(1, 0.0, 1)
     m = [local.mesh(V, T, F.RSS), local.mesh(*F.icosphere(1, 0.15, 2), F.RSS)]
     local.mesh_refit(m[0], torch.from_numpy(V * 0.1).to(DEV), bottomup=True)
@@ -91,9 +96,11 @@ def test_distance_over_merged_bvs(n):
     local.close()
 
 
-@pytest.mark.parametrize("n", [BLOCKS + 77, PAST])
-def test_mesh_against_primitives(ctx, poses, n):
-    print("case: %d mesh-shape queries" % n, flush=True)
+@pytest.mark.parametrize("n,lanes", [(BLOCKS + 77, 1), (PAST, 1), (PAST, 2)])
+def test_mesh_against_primitives(poses, n, lanes):
+    print("case: %d mesh-shape queries, lanes=%d" % (n, lanes), flush=True)
+    ctx = F.Context(0)
+    ctx.set_engine_param("ordered_lanes", lanes)
     mesh = ctx.mesh(*F.icosphere(4, 0.15, 1))
     rec, pool = F.shape_table([F.BOX], [(0.6, 0.4, 0.5)])
     shapes = torch.from_numpy(np.ascontiguousarray(rec).view(np.uint8)).to(DEV)
@@ -112,6 +119,7 @@ def test_mesh_against_primitives(ctx, poses, n):
     want = run(PERIOD).cpu().numpy()
     assert 0 < want.mean() < 1
     assert _repeats(run(n), want)
+    ctx.close()
 
 
 @pytest.mark.parametrize("n", [(1 << 24) + 5, 1 << 28])
