@@ -56,6 +56,18 @@ hipError_t dmalloc(T** p, size_t n) {
   return hipMalloc(reinterpret_cast<void**>(p), sizeof(T) * std::max<size_t>(n, 1));
 }
 
+// Device memory of `record` elements for each of at least `want` records.
+template <typename T>
+hipError_t grow_records(T** p, long long* have, long long want, size_t record) {
+  if (want <= *have) return hipSuccess;
+  (void)hipFree(*p);
+  *p = nullptr;
+  *have = 0;
+  const hipError_t e = dmalloc(p, record * static_cast<size_t>(want));
+  if (e == hipSuccess) *have = want;
+  return e;
+}
+
 __global__ void clear_fronts(int32_t* sizes, int32_t* meshes, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -86,6 +98,7 @@ struct SingleIo {
   long long tests[2];
   double distance[7];  // and the two nearest points
 };
+constexpr long long kSinglePinned = 4096;  // records of a call in pinned memory
 
 }  // namespace
 
@@ -100,9 +113,13 @@ struct fclx_context {
   hipStream_t stream = nullptr;  // single-query calls
   // single-query staging
   SingleIo* one = nullptr;
-  int32_t* s_pairs = nullptr;    // pinned, s_pairs_cap records
-  double* s_geo = nullptr;       // pinned contact geometry: 7 doubles per record
-  long long s_pairs_cap = 0;
+  // records of collide(): the first kSinglePinned pinned, which the kernel
+  // writes over the link; a call that finds more repeats into device memory
+  int32_t* s_pairs = nullptr;
+  double* s_geo = nullptr;       // 7 doubles per record, once a call asks for geometry
+  int32_t* s_many_pairs = nullptr;  // device, s_many_cap records
+  double* s_many_geo = nullptr;     // device, s_many_geo_cap records
+  long long s_many_cap = 0, s_many_geo_cap = 0;
   int32_t* s_status = nullptr;   // device status word of the single-query calls
   EngineWorkspace* ws = nullptr;
   std::mutex ws_mu;       // the FAST engine's work buffers (one batch at a time)
@@ -304,6 +321,8 @@ void fclx_shutdown(fclx_context* ctx) {
   if (ctx->one) (void)hipHostFree(ctx->one);
   if (ctx->s_pairs) (void)hipHostFree(ctx->s_pairs);
   if (ctx->s_geo) (void)hipHostFree(ctx->s_geo);
+  (void)hipFree(ctx->s_many_pairs);
+  (void)hipFree(ctx->s_many_geo);
   (void)hipFree(ctx->s_status);
   (void)hipFree(ctx->s_shape);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -1117,6 +1136,11 @@ int fclx_get_engine_param(fclx_context* ctx, const char* name, double* value) {
     *value = ctx->shape_waves;
   } else if (n == "serve_fail_launches") {
     *value = ctx->serve_fail_launches.load();
+  } else if (n == "single_pinned_bytes") {
+    std::lock_guard<std::mutex> sl(ctx->mu);
+    *value = static_cast<double>(sizeof(SingleIo) +
+                                 (ctx->s_pairs ? 3 * sizeof(int32_t) * kSinglePinned : 0) +
+                                 (ctx->s_geo ? 7 * sizeof(double) * kSinglePinned : 0));
   } else {
     return fail(ctx, FCLX_ERR_INVALID_ARGUMENT, "unknown engine parameter");
   }
@@ -1429,22 +1453,25 @@ int collide_one(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_t 
   const int depth_sum = ctx->meshes[mesh1].bvh.depth + ctx->meshes[mesh2].bvh.depth;
   if (depth_sum > kMaxStack)
     return fail(ctx, FCLX_ERR_UNSUPPORTED, "hierarchy deeper than the traversal stack bound");
-  // staging for the records starts small and grows to the count found
-  long long want = std::min<long long>(cap, 4096);
   SingleIo& io = *ctx->one;
+  if (!ctx->s_pairs)
+    HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->s_pairs),
+                               3 * sizeof(int32_t) * kSinglePinned));
+  if (contact && !ctx->s_geo)
+    HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->s_geo),
+                               7 * sizeof(double) * kSinglePinned));
+  int32_t* rec = ctx->s_pairs;
+  double* geo = ctx->s_geo;
+  long long room = kSinglePinned;
+  // a cap beyond the pinned room after a call that needed more: at once into
+  // device memory, or each such call would run twice
+  const long long many = contact ? std::min(ctx->s_many_cap, ctx->s_many_geo_cap) : ctx->s_many_cap;
+  if (cap > kSinglePinned && many > kSinglePinned) {
+    rec = ctx->s_many_pairs;
+    geo = ctx->s_many_geo;
+    room = many;
+  }
   for (int attempt = 0; attempt < 2; ++attempt) {
-    if (want > ctx->s_pairs_cap) {
-      if (ctx->s_pairs) (void)hipHostFree(ctx->s_pairs);
-      if (ctx->s_geo) (void)hipHostFree(ctx->s_geo);
-      ctx->s_pairs = nullptr;
-      ctx->s_geo = nullptr;
-      ctx->s_pairs_cap = 0;
-      HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->s_pairs),
-                                 3 * sizeof(int32_t) * static_cast<size_t>(want)));
-      HIP_TRY(ctx, hipHostMalloc(reinterpret_cast<void**>(&ctx->s_geo),
-                                 7 * sizeof(double) * static_cast<size_t>(want)));
-      ctx->s_pairs_cap = want;
-    }
     CollideLaunch L{};
     L.meshes = ctx->d_table;
     L.num_meshes = static_cast<int32_t>(ctx->meshes.size());
@@ -1454,22 +1481,27 @@ int collide_one(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_t 
     L.tf2 = io.tf + 12;
     L.cap = cap;
     L.counts = &io.count;
-    L.pairs = ctx->s_pairs;
-    L.pair_capacity = ctx->s_pairs_cap;
+    L.pairs = rec;
+    L.pair_capacity = room;
     L.bv_tests = io.tests;
     L.leaf_tests = io.tests + 1;
     L.status = ctx->s_status;
     L.carry_max = ctx->ordered_carry_max.load();
     if (contact) {
       L.contact = 1;
-      L.contact_pos = ctx->s_geo;
-      L.contact_normal = ctx->s_geo + 3 * ctx->s_pairs_cap;
-      L.contact_depth = ctx->s_geo + 6 * ctx->s_pairs_cap;
+      L.contact_pos = geo;
+      L.contact_normal = geo + 3 * room;
+      L.contact_depth = geo + 6 * room;
     }
     HIP_TRY(ctx, launch_collide_ordered(L, depth_sum, s));
     HIP_TRY(ctx, hipStreamSynchronize(s));
-    if (io.count <= ctx->s_pairs_cap) break;
-    want = io.count;  // every contact of this query fits on the second run
+    if (std::min(io.count, capacity) <= room) break;
+    // every contact of this query fits on the second run
+    room = io.count;
+    HIP_TRY(ctx, grow_records(&ctx->s_many_pairs, &ctx->s_many_cap, room, 3));
+    if (contact) HIP_TRY(ctx, grow_records(&ctx->s_many_geo, &ctx->s_many_geo_cap, room, 7));
+    rec = ctx->s_many_pairs;
+    geo = ctx->s_many_geo;
   }
   const int32_t count = io.count;
   *num_contacts = count;
@@ -1479,15 +1511,31 @@ int collide_one(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_t 
   }
   const int32_t ncopy = std::min(count, capacity);
   if (ncopy > 0) {
+    const size_t n = static_cast<size_t>(ncopy);
+    const bool on_device = room > kSinglePinned;
+    std::vector<int32_t> copied;
+    if (on_device) {
+      copied.resize(3 * n);
+      HIP_TRY(ctx, hipMemcpy(copied.data(), rec, sizeof(int32_t) * 3 * n, hipMemcpyDeviceToHost));
+      rec = copied.data();
+    }
     for (int i = 0; i < ncopy; ++i) {
-      pairs[2 * i] = ctx->s_pairs[3 * i + 1];
-      pairs[2 * i + 1] = ctx->s_pairs[3 * i + 2];
+      pairs[2 * i] = rec[3 * i + 1];
+      pairs[2 * i + 1] = rec[3 * i + 2];
     }
     if (contact) {
-      const size_t n = static_cast<size_t>(ncopy), room = static_cast<size_t>(ctx->s_pairs_cap);
-      std::memcpy(pos, ctx->s_geo, 3 * sizeof(double) * n);
-      std::memcpy(normal, ctx->s_geo + 3 * room, 3 * sizeof(double) * n);
-      std::memcpy(depth, ctx->s_geo + 6 * room, sizeof(double) * n);
+      struct Part {
+        double* to;
+        const double* from;
+        size_t count;
+      };
+      for (const Part& p : {Part{pos, geo, 3 * n}, Part{normal, geo + 3 * room, 3 * n},
+                            Part{depth, geo + 6 * room, n}}) {
+        if (on_device)
+          HIP_TRY(ctx, hipMemcpy(p.to, p.from, sizeof(double) * p.count, hipMemcpyDeviceToHost));
+        else
+          std::memcpy(p.to, p.from, sizeof(double) * p.count);
+      }
     }
   }
   if (count > capacity)

@@ -439,7 +439,8 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               kernel (default 2)
  * Results do not depend on them; smaller buffers mean more rounds. */
 int fclx_set_engine_param(fclx_context* ctx, const char* name, double value);
-/* The current value of a tunable above (for tuners); no reference
+/* The current value of a tunable above, or "single_pinned_bytes": page-locked
+ * host memory held for the single-query calls (for tuners and tests); no reference
  * counterpart. */
 int fclx_get_engine_param(fclx_context* ctx, const char* name, double* value);
 int fclx_engine_last_report(fclx_context* ctx, fclx_engine_report* out);

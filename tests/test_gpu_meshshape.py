@@ -166,16 +166,19 @@ def chain_mesh(n, s=0.05):
     return V, T, xs
 
 
-def test_mesh_shape_deep_hierarchy():
+@pytest.mark.parametrize("list_depth", [440, 71])
+def test_mesh_shape_deep_hierarchy(list_depth):
     """A mesh 72 levels deep (a chain of triangles that the mean split
-    peels off one at a time): the descent stack leaves LDS for device
-    memory and every count, triangle, statistic and contact equals the
-    oracle's.  Own context: a deep mesh switches every mesh-shape batch of
-    its context to the device-memory stack."""
+    peels off one at a time): within the depth of the wavefronts' lists in LDS,
+    and beyond a lowered one, where every mesh-shape batch of the context keeps
+    its descent stacks in device memory.  Every count, triangle, statistic and
+    contact equals the oracle's.  (Each level multiplies the chain's length by
+    twice the triangles left, so in doubles no chain comes near the 440.)"""
     V, T, xs = chain_mesh(72)
     depth = F.bvh_build(V, T)["depth"]
     assert depth == 72, depth
     c2 = F.Context(0)
+    c2.set_engine_param("meshshape_list_depth", list_depth)
     try:
         mid = c2.mesh(V, T)
         assert c2.mesh_info(mid)["depth"] == depth

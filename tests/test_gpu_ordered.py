@@ -194,3 +194,38 @@ def test_light_contexts(n, meshes):
     _same(local, qm, tf1, tf2, 1, True)
     _same(local, qm, tf1, tf2, 5, True)
     local.close()
+
+
+def test_single_calls_with_many_contacts():
+    """More records than a call's pinned room: through device memory, the
+    page-locked memory stays as it is, and small answers follow large ones."""
+    print("case: single calls with many contacts", flush=True)
+    local = F.Context(0)
+    A, B = F.icosphere(32, 0.05, 9), F.icosphere(32, 0.05, 10)
+    m = [local.mesh(*A), local.mesh(*B)]
+    I = np.array([1, 0, 0, 0, 1, 0, 0, 0, 1, 0, 0, 0], float)
+    near, far = I.copy(), I.copy()
+    near[9:], far[9:] = [0.02, 0.01, 0.03], [1.8, 0.3, 0.1]
+    rc, counts, per_q, bv, leaf, _ = collide_gpu(local, np.array([m], np.int32), I[None],
+                                                 near[None], 10**6, capacity=1 << 20)
+    full = per_q[0]
+    assert rc == 0 and len(full) == counts[0] > 3 * 4096
+    held = None
+    for cap in (4095, 4096, 4097, 10**6, 100, 10**6):
+        pairs, stats = local.collide(m[0], I, m[1], near, cap=cap)
+        assert np.array_equal(pairs, full[:cap])
+        few = local.collide(m[0], I, m[1], far, cap=cap)[0]
+        assert len(few) < 1000
+        if cap > len(full):
+            assert stats.tolist() == [bv[0], leaf[0]]
+        held = held or local.get_engine_param("single_pinned_bytes")
+    assert local.get_engine_param("single_pinned_bytes") == held < 4096 * 12 + 1024
+    # the geometry of a small answer (pinned) begins that of a large one
+    small = local.collide_contact(m[0], I, m[1], near, cap=3000)
+    large = local.collide_contact(m[0], I, m[1], near, cap=10**6)
+    again = local.collide_contact(m[0], I, m[1], near, cap=10**6)
+    assert len(small[0]) == 3000 and len(large[0]) > 4096
+    for a, b, c in zip(small[:4], large[:4], again[:4]):
+        assert np.array_equal(a, b[:3000]) and np.array_equal(b, c)
+    assert local.get_engine_param("single_pinned_bytes") < 4096 * 68 + 1024
+    local.close()
