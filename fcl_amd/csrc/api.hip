@@ -128,6 +128,7 @@ struct fclx_context {
   char* s_shape = nullptr;        // single shape-pair staging (under mu)
   size_t s_shape_bytes = 0;
   int epa_blocks_per_cu = 0;
+  int epa_lanes_min = kEpaLanesMin;
   int shape_waves = 2;
   std::atomic<int> serve_fail_launches{0};  // failure injection for the serving loop
   std::atomic<uint32_t> ordered_carry_max{1u << 31};
@@ -965,6 +966,7 @@ int fclx_shape_collide_batch(fclx_context* ctx, const fclx_shape_collide_batch_a
   std::lock_guard<std::mutex> lock(ctx->sws_mu);
   if (!ctx->sws) ctx->sws = shape_workspace_create(ctx->device);
   shape_workspace_set_epa_blocks_per_cu(ctx->sws, ctx->epa_blocks_per_cu);
+  shape_workspace_set_epa_lanes_min(ctx->sws, ctx->epa_lanes_min);
   shape_workspace_set_waves(ctx->sws, ctx->shape_waves);
   ShapeLaunch L{};
   L.num_pairs = a->num_pairs;
@@ -1063,6 +1065,7 @@ int fclx_shape_collide(fclx_context* ctx, const fclx_shape* s1, const double* ve
     std::lock_guard<std::mutex> sl(ctx->sws_mu);
     if (!ctx->sws) ctx->sws = shape_workspace_create(ctx->device);
     shape_workspace_set_epa_blocks_per_cu(ctx->sws, ctx->epa_blocks_per_cu);
+    shape_workspace_set_epa_lanes_min(ctx->sws, ctx->epa_lanes_min);
     shape_workspace_set_waves(ctx->sws, ctx->shape_waves);
     hipError_t e = shape_collide_run(ctx->sws, L, ctx->stream);
     if (e != hipSuccess) return hip_fail(ctx, e, "shape collide launch");
@@ -1131,6 +1134,9 @@ int fclx_get_engine_param(fclx_context* ctx, const char* name, double* value) {
   else if (n == "epa_blocks_per_cu") {
     std::lock_guard<std::mutex> sl(ctx->sws_mu);
     *value = ctx->epa_blocks_per_cu;
+  } else if (n == "epa_lanes_min") {
+    std::lock_guard<std::mutex> sl(ctx->sws_mu);
+    *value = ctx->epa_lanes_min;
   } else if (n == "shape_waves_per_simd") {
     std::lock_guard<std::mutex> sl(ctx->sws_mu);
     *value = ctx->shape_waves;
@@ -1213,6 +1219,9 @@ int fclx_set_engine_param(fclx_context* ctx, const char* name, double value) {
   } else if (n == "epa_blocks_per_cu" && in(0, 32)) {
     std::lock_guard<std::mutex> sl(ctx->sws_mu);
     ctx->epa_blocks_per_cu = static_cast<int>(value);
+  } else if (n == "epa_lanes_min" && in(1, 2147483647.0)) {
+    std::lock_guard<std::mutex> sl(ctx->sws_mu);
+    ctx->epa_lanes_min = static_cast<int>(value);
   } else if (n == "shape_waves_per_simd" && in(2, 4)) {
     std::lock_guard<std::mutex> sl(ctx->sws_mu);
     ctx->shape_waves = static_cast<int>(value);

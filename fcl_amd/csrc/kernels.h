@@ -213,13 +213,16 @@ struct RefitLaunch {
 // level_offsets_host[l] .. [l+1] (host array of levels + 1) bounding each.
 hipError_t launch_refit(const RefitLaunch& L, bool bottomup, const int32_t* level_nodes,
                         const int32_t* level_offsets_host, int levels, hipStream_t s);
-// Sort buffers and the EPA queue of the shape path; one
-// per context, used by one batch at a time (the caller serialises calls;
-// batches on different streams are ordered through an event).
+// Sort buffers, the EPA queue and, once a batch of kEpaLanesMin pairs asked for
+// contacts, the polytopes of its lanes (1.5 GB); one per context, used by one
+// batch at a time (the caller serialises calls; batches on different streams
+// are ordered through an event).
+constexpr int kEpaLanesMin = 240000;
 struct ShapeWorkspace;
 ShapeWorkspace* shape_workspace_create(int device);
 void shape_workspace_destroy(ShapeWorkspace* w);
 void shape_workspace_set_epa_blocks_per_cu(ShapeWorkspace* w, int blocks);
+void shape_workspace_set_epa_lanes_min(ShapeWorkspace* w, int pairs);
 void shape_workspace_set_waves(ShapeWorkspace* w, int waves);
 hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_t s);
 hipError_t launch_distance_plain(const DistanceLaunch& L, int stack_need, hipStream_t s);

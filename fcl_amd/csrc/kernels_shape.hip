@@ -16,7 +16,8 @@
 //   3. EPA over the queue (GJK's final simplex per pair): a persistent grid
 //      of lane groups, each with one pair's polytope in LDS, taking the next
 //      pair when done; then the pairs whose polytopes outgrew those stores,
-//      from the start, in stores of the reference's full size.
+//      from the start, in stores of the reference's full size.  Long queues
+//      run a lane per pair instead, its polytope in device memory.
 // Same-address atomics are kept few: one per block per counter in the
 // sorting and GJK kernels (the GJK kernel's on per-XCD counters), one per
 // wavefront's idle groups in EPA.
@@ -285,13 +286,14 @@ __global__ void __launch_bounds__(kBlk, kWaves) shape_gjk(ShapeLaunch L, const i
 // pair the polytopes (11.6 KB each, 131,072 of them) were in device memory,
 // and the walk's scattered reads moved whole lines from HBM.  1,000,000 pairs
 // (200,000 of them in here): 7.5 ms -> 4.6 + 1.8; the whole call 8.7 -> 7.7 ms
-// for 1,000,000 pairs, 5.1 -> 1.8 for 100,000, 2.7 -> 1.1 for 1,000.
+// for 1,000,000 pairs, 5.1 -> 1.8 for 100,000, 2.7 -> 1.1 for 1,000.  Longer
+// queues (lanes_min) are for shape_epa_lanes.
 template <typename Store, int G>
 __global__ void __launch_bounds__(shp::kEpaBlock, 2) shape_epa(ShapeLaunch L,
                                                                const shp::EpaSeed* seeds,
                                                                int32_t* ctr, int sub_cap,
                                                                const int32_t* todo,
-                                                               int32_t* spill) {
+                                                               int32_t* spill, int lanes_min) {
   __shared__ Store stores[shp::kEpaBlock / G];
   struct Job {
     const ShapeLaunch& L;
@@ -343,8 +345,116 @@ __global__ void __launch_bounds__(shp::kEpaBlock, 2) shape_epa(ShapeLaunch L,
     total += ctr[kCtrQueue + x];
     job.sub_end[x] = total;
   }
+  if (total >= lanes_min) return;  // shape_epa_lanes has them
   if (todo) total = ctr[kCtrSpill];
   shp::epa_groups<G>(job, stores, total, &ctr[todo ? kCtrSpillGrab : kCtrGrab], L.tol);
+}
+
+// Idle lanes of a wavefront take new pairs once this many are idle (or all).
+constexpr int kRefill = 16;
+
+// EPA over the queued pairs (the sub-queues, concatenated), a lane each with its
+// polytope in device memory, for queues of lanes_min pairs or more.  A
+// wavefront takes 64 entries at a time with one atomic; every lane runs its
+// own pair one loop pass per trip and takes the wavefront's next entry when
+// done, so lanes do not wait for the slowest pair of their wavefront.
+//
+// Bound: the horizon walk's scattered reads of the polytopes (11.6 KB a lane,
+// 131,072 lanes), which move whole lines from HBM, and below the line the
+// longest pair of one lane (2.5 ms).  The lane groups of shape_epa do not wait
+// for memory, but repeat each walk in 16 lanes: their time per pair is larger.
+// Whole batches, lanes / groups, by EPA pairs: mixed kinds 20,000 4.7 / 1.8 ms,
+// 202,000 8.2 / 7.7, 302,000 11.0 / 11.1, 804,000 24.5 / 27.8; cylinders 99,000
+// 4.5 / 3.7, 248,000 7.6 / 7.9, 991,000 23.5 / 29.5; convexes of 32 points
+// 100,000 2.9 / 2.5, 250,000 4.7 / 5.0, 1,000,000 14.1 / 18.3.
+__global__ void __launch_bounds__(kBlk, 2) shape_epa_lanes(ShapeLaunch L,
+                                                           const shp::EpaSeed* seeds,
+                                                           int32_t* ctr, int sub_cap,
+                                                           shp::EpaLane* lanes,
+                                                           shp::EpaWave* waves, int lanes_min) {
+  const int lane = threadIdx.x & 63;
+  const size_t gid = static_cast<size_t>(blockIdx.x) * kBlk + threadIdx.x;
+  int sub_end[8];  // running totals of the sub-queue sizes
+  int total = 0;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) {
+    total += ctr[kCtrQueue + x];
+    sub_end[x] = total;
+  }
+  if (total < lanes_min) return;
+  const int wid = static_cast<int>(gid / 64);
+  int cursor = 0, stop = 0;  // the wavefront's entries not yet started
+  bool exhausted = false;
+  // the horizon walk's stack in LDS, one column per thread (a frame is
+  // popped right after the walk returns from a child, at LDS latency)
+  __shared__ int16_t xs_lds[shp::kNfEpa][kBlk];
+  shp::Epa E;
+  E.M = lanes + gid;
+  E.S = waves + wid;
+  E.lane = lane;
+  E.xs = &xs_lds[0][threadIdx.x];
+  E.xs_stride = kBlk;
+  shp::MDiff m;
+  int q = -1, gjk_passes = 0;
+  bool active = false;
+  while (true) {
+    bool finish = false, started = false;
+    const unsigned long long idle = __ballot(!active);
+    const int nidle = __popcll(idle);
+    if (cursor >= stop && !exhausted && (nidle == 64 || nidle >= kRefill)) {
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&ctr[kCtrGrab], 64);
+      base = __shfl(base, 0);
+      cursor = base < total ? base : total;
+      stop = base + 64 < total ? base + 64 : total;
+      exhausted = base + 64 >= total;
+    }
+    if (cursor < stop && (nidle == 64 || nidle >= kRefill)) {
+      const int v = cursor + __popcll(idle & ((1ull << lane) - 1));
+      cursor = cursor + nidle < stop ? cursor + nidle : stop;
+      if (!active && v < stop) {
+        int x = 0, before = 0;
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+          if (v >= sub_end[k]) {
+            x = k + 1;
+            before = sub_end[k];
+          }
+        const shp::EpaSeed& sd = seeds[static_cast<size_t>(x) * sub_cap + (v - before)];
+        q = sd.q;
+        gjk_passes = sd.gjk_passes;
+        shp::Shape s1, s2;
+        load_shape(L, L.pair_shapes[2 * q], s1);
+        load_shape(L, L.pair_shapes[2 * q + 1], s2);
+        shp::make_mdiff(s1, shp::xf_load(L.tf1 + 12 * static_cast<size_t>(q)), s2,
+                        shp::xf_load(L.tf2 + 12 * static_cast<size_t>(q)), m);
+        shp::Gjk g;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          g.w[k] = sd.w[k];
+          g.d[k] = sd.d[k];
+        }
+        g.rank = sd.rank;
+        active = shp::epa_start(E, g, m, L.tol);
+        finish = !active;
+        started = true;
+      }
+    }
+    if (active && !started) {
+      active = shp::epa_step(E, m, L.tol);
+      finish = !active;
+    }
+    if (finish) {
+      const shp::Contact c =
+          shp::epa_finish(E, m, shp::xf_load(L.tf1 + 12 * static_cast<size_t>(q)));
+      write_contacts(L, q, &c, 1);
+      if (L.passes) {
+        L.passes[2 * q] = gjk_passes;
+        L.passes[2 * q + 1] = E.fallback ? 0 : E.it;
+      }
+    }
+    if (exhausted && cursor >= stop && !__ballot(active)) break;
+  }
 }
 
 }  // namespace
@@ -357,6 +467,10 @@ struct ShapeWorkspace {
   shp::EpaSeed* seeds = nullptr;  // EPA queue (allocated with enable_contact)
   long long seed_cap = 0;
   int32_t* ctr = nullptr;
+  shp::EpaLane* epa = nullptr;  // polytopes of shape_epa_lanes, once a batch could need them
+  shp::EpaWave* epa_waves = nullptr;
+  int epa_lane_blocks = 0;
+  int epa_lanes_min = kEpaLanesMin;  // EPA queues from this size on: a lane per pair
   int epa_blocks_per_cu = 0;  // 0: as many as fit
   int waves = 2;              // register budget of the GJK kernel (waves per SIMD)
   hipEvent_t done = nullptr;
@@ -385,6 +499,8 @@ void shape_workspace_destroy(ShapeWorkspace* w) {
   if (w->pending) (void)hipEventSynchronize(w->done);
   release_buffers(w);
   (void)hipFree(w->ctr);
+  (void)hipFree(w->epa);
+  (void)hipFree(w->epa_waves);
   if (w->done) (void)hipEventDestroy(w->done);
   delete w;
 }
@@ -392,6 +508,8 @@ void shape_workspace_destroy(ShapeWorkspace* w) {
 void shape_workspace_set_epa_blocks_per_cu(ShapeWorkspace* w, int blocks) {
   w->epa_blocks_per_cu = blocks;
 }
+
+void shape_workspace_set_epa_lanes_min(ShapeWorkspace* w, int pairs) { w->epa_lanes_min = pairs; }
 
 void shape_workspace_set_waves(ShapeWorkspace* w, int waves) { w->waves = waves; }
 
@@ -441,6 +559,21 @@ hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_
     w->cap = cap;
     w->seed_cap = seed_cap;
   }
+  const bool epa_lanes = L.contact && n >= w->epa_lanes_min;
+  if (epa_lanes && w->epa_lane_blocks < epa_blocks) {
+    if (w->pending && (e = hipEventSynchronize(w->done)) != hipSuccess) return e;
+    w->pending = false;
+    (void)hipFree(w->epa);
+    (void)hipFree(w->epa_waves);
+    w->epa = nullptr;
+    w->epa_waves = nullptr;
+    w->epa_lane_blocks = 0;
+    const size_t lanes = static_cast<size_t>(epa_blocks) * kBlk;
+    if ((e = hipMalloc(&w->epa, sizeof(shp::EpaLane) * lanes)) != hipSuccess ||
+        (e = hipMalloc(&w->epa_waves, sizeof(shp::EpaWave) * (lanes / 64))) != hipSuccess)
+      return e;
+    w->epa_lane_blocks = epa_blocks;
+  }
   // a batch on another stream may still be using the buffers
   if (w->pending && (e = hipStreamWaitEvent(s, w->done, 0)) != hipSuccess) return e;
 
@@ -454,9 +587,12 @@ hipError_t shape_collide_run(ShapeWorkspace* w, const ShapeLaunch& L, hipStream_
   if (L.contact) {
     // (the sorted positions are done with: their array takes the spilled entries)
     shape_epa<shp::EpaSmall, shp::kEpaSmallLanes><<<epa_blocks, shp::kEpaBlock, 0, s>>>(
-        L, w->seeds, w->ctr, sub_cap, nullptr, w->perm);
+        L, w->seeds, w->ctr, sub_cap, nullptr, w->perm, w->epa_lanes_min);
     shape_epa<shp::EpaLarge, shp::kEpaLargeLanes><<<epa_blocks, shp::kEpaBlock, 0, s>>>(
-        L, w->seeds, w->ctr, sub_cap, w->perm, nullptr);
+        L, w->seeds, w->ctr, sub_cap, w->perm, nullptr, w->epa_lanes_min);
+    if (epa_lanes)
+      shape_epa_lanes<<<epa_blocks, kBlk, 0, s>>>(L, w->seeds, w->ctr, sub_cap, w->epa,
+                                                  w->epa_waves, w->epa_lanes_min);
   }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if ((e = hipEventRecord(w->done, s)) != hipSuccess) return e;

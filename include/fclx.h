@@ -435,6 +435,10 @@ int fclx_set_profiling(fclx_context* ctx, int32_t enable);
  *                               on MI355X)
  *   "epa_blocks_per_cu" 0..32   most blocks per CU of the shape path's EPA
  *                               kernels (0: the two that LDS has room for)
+ *   "epa_lanes_min"     1..2^31-1  EPA pairs of a shape batch from which they
+ *                               run a lane each, in 1.5 GB of device memory
+ *                               that the context then keeps, instead of by
+ *                               lane groups in LDS (default 240000)
  *   "shape_waves_per_simd" 2..4 register budget of the shape path's GJK
  *                               kernel (default 2)
  * Results do not depend on them; smaller buffers mean more rounds. */

@@ -27,6 +27,20 @@ def _curved(n, seed, flat):
     return rec, pool, ps, W.random_poses(n, rng, 0.25), W.random_poses(n, rng, 0.25)
 
 
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("n", [1, 65, 2000])
+def test_long_queues_run_a_lane_each(ctx, n, over):
+    """On both sides of the queue length from which EPA runs a lane per pair."""
+    rec, pool, ps, tf1, tf2 = _curved(n, 11 * n, 1.0)
+    queue = int((fclo.shape_collide_batch(fclo.shapes_from_table(rec, pool), ps, tf1, tf2, 1, True,
+                                          passes=True)[2][:, 1] > 0).sum())
+    ctx.set_engine_param("epa_lanes_min", max(queue, 1) + over)
+    try:
+        check_parity(ctx, rec, pool, ps, tf1, tf2, 1, True, "lanes from %d EPA pairs" % (queue + over))
+    finally:
+        ctx.set_engine_param("epa_lanes_min", 240000)
+
+
 @pytest.mark.parametrize("n", [1, 2, 15, 17, 33, 257, 6000])
 @pytest.mark.parametrize("flat", [1.0, 0.02])
 def test_small_and_full_stores(ctx, n, flat):
