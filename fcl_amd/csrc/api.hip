@@ -706,6 +706,7 @@ int collide_batch_status(fclx_context* ctx, const fclx_collide_batch_args* a, vo
   L.leaf_tests = reinterpret_cast<long long*>(a->leaf_tests);
   L.status = d_status;
   L.carry_max = ctx->ordered_carry_max.load();
+  L.node_pairs_max = static_cast<long long>(nodes) * static_cast<long long>(nodes);
   L.lanes_max = lanes_max(ctx, collide_lanes_max(a->num_queries, a->num_max_contacts, nodes_min,
                                                  nodes));
   hipError_t e;
@@ -936,7 +937,6 @@ int fclx_mesh_shape_collide_batch(fclx_context* ctx, const fclx_mesh_shape_colli
   L.contact_depth = a->contact_depth;
   L.stats = reinterpret_cast<long long*>(a->stats);
   L.status = ctx->d_status;
-  L.carry_max = ctx->ordered_carry_max.load();
   L.lanes_max = lanes_max(ctx, mesh_shape_lanes_max(a->num_queries, a->num_max_contacts, nodes_min,
                                                     nodes));
   L.list_depth = ctx->meshshape_list_depth.load();
@@ -1496,6 +1496,8 @@ int collide_one(fclx_context* ctx, int32_t mesh1, const double tf1[12], int32_t 
     L.leaf_tests = io.tests + 1;
     L.status = ctx->s_status;
     L.carry_max = ctx->ordered_carry_max.load();
+    L.node_pairs_max = static_cast<long long>(ctx->meshes[mesh1].bvh.nodes.size()) *
+                       static_cast<long long>(ctx->meshes[mesh2].bvh.nodes.size());
     if (contact) {
       L.contact = 1;
       L.contact_pos = geo;

@@ -50,6 +50,7 @@ struct CollideLaunch {
   // world-frame point (3), normal (3) and penetration depth
   int32_t contact;
   uint32_t carry_max;          // ordered kernel: most BV tests its list carries
+  long long node_pairs_max;    // no query has more node pairs (nor BV tests)
   double* contact_pos;
   double* contact_normal;
   double* contact_depth;
@@ -134,7 +135,6 @@ struct MeshShapeLaunch {
   int32_t* status;
   int32_t leaf_share;           // percent of a wavefront's lanes with a leaf that starts a
                                 // leaf round (1..100; 0: 100)
-  uint32_t carry_max;           // most BV tests that a query's list carries
   int32_t list_depth;           // at most kMsListDepth (lower in tests)
   size_t epa_queue;             // at most kMsEpaQueue (lower in tests)
   long long lanes_max;          // queries on meshes of at most this many nodes run on a lane

@@ -546,7 +546,7 @@ __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery*
   constexpr int G = 64, kCap = kMsListCap;
   const LaneGroup<G> g;
   if (queries[q].valid == 0) return;
-  OrdTotals T = ord_begin(g, S, L.carry_max);
+  OrdTotals T = ord_begin(g, S, 0u);
   if (g.lane == 0) {
     const MeshDev& M = L.meshes[L.query_meshes[q]];
     (void)load_query(L, static_cast<int>(q), w.s, L.max_depth);
@@ -576,9 +576,8 @@ __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery*
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   while (T.sp > 0) {
-    int n = ord_window<G, kCap>(T.sp, margin);
-    if constexpr (kStats)
-      if (--T.audit_in < 0) ord_audit(g, S, T, L.carry_max, n);
+    // (a query tests no node twice: its counts fit the list's 32 bits)
+    const int n = ord_window<G, kCap>(T.sp, margin);
     const bool on = g.lane < n;
     unsigned long long e = 0;
     uint2 acc = make_uint2(0u, 0u);
@@ -685,20 +684,26 @@ __device__ __forceinline__ void descend(const MeshShapeLaunch& L, const MsQuery*
   }
 }
 
-template <bool kStats, bool kContact, int kWaves>
+// A block per query from `first` on (a loop over queries took 1 % of a batch);
+// kSome: the last part of an order, whose other queries are the lanes'.
+template <bool kStats, bool kContact, int kWaves, bool kSome>
 __global__ void __launch_bounds__(64, kWaves) meshshape_ordered(MeshShapeLaunch L,
                                                                 const MsQuery* queries, int margin,
                                                                 int leaf_min, MsEpaSeed* seeds,
                                                                 unsigned long long* nseed,
-                                                                const int32_t* order,
+                                                                int first, const int32_t* order,
                                                                 const int32_t* ctr) {
   __shared__ OrderedList<kMsListCap, kStats> S;
   __shared__ MsWave w;
-  // all queries, or the order's last part
-  const size_t end = L.num_queries, first = order ? end - static_cast<size_t>(ctr[6]) : 0;
-  for (size_t k = first + blockIdx.x; k < end; k += gridDim.x)
-    descend<kStats, kContact>(L, queries, order ? static_cast<size_t>(order[k]) : k, margin,
-                              leaf_min, seeds, nseed, S, w);
+  if constexpr (kSome) {
+    const size_t end = L.num_queries;
+    for (size_t k = end - static_cast<size_t>(ctr[6]) + blockIdx.x; k < end; k += gridDim.x)
+      descend<kStats, kContact>(L, queries, static_cast<size_t>(order[k]), margin, leaf_min, seeds,
+                                nseed, S, w);
+  } else {
+    descend<kStats, kContact>(L, queries, static_cast<size_t>(first) + blockIdx.x, margin, leaf_min,
+                              seeds, nseed, S, w);
+  }
 }
 
 // A query per lane.  Lanes of a wavefront step together: a lane whose descent
@@ -973,17 +978,25 @@ __global__ void ms_zero_u64(unsigned long long* p) {
 
 namespace {
 
-template <int kWaves>
+template <int kWaves, bool kSome>
 void launch_descent(const MeshShapeLaunch& L, const MsQuery* queries, MsEpaSeed* seeds,
                     unsigned long long* nseed, const int32_t* order, const int32_t* ctr,
                     hipStream_t s) {
-  auto kernel = L.contact ? (L.stats ? meshshape_ordered<true, true, kWaves>
-                                     : meshshape_ordered<false, true, kWaves>)
-                          : (L.stats ? meshshape_ordered<true, false, kWaves>
-                                     : meshshape_ordered<false, false, kWaves>);
+  auto kernel = L.contact ? (L.stats ? meshshape_ordered<true, true, kWaves, kSome>
+                                     : meshshape_ordered<false, true, kWaves, kSome>)
+                          : (L.stats ? meshshape_ordered<true, false, kWaves, kSome>
+                                     : meshshape_ordered<false, false, kWaves, kSome>);
   const int leaf_min = L.leaf_share > 0 ? std::max(1, 64 * L.leaf_share / 100) : 64;
-  kernel<<<group_blocks(L.num_queries), 64, 0, s>>>(L, queries, L.max_depth + 2, leaf_min, seeds,
-                                                    nseed, order, ctr);
+  // HIP refuses a launch of 2^32 threads
+  constexpr int kPart = 1 << 25;
+  for (long long first = 0; first < L.num_queries; first += kPart) {
+    const long long left = L.num_queries - first;
+    const unsigned blocks =
+        kSome ? group_blocks(left) : static_cast<unsigned>(std::min<long long>(left, kPart));
+    kernel<<<blocks, 64, 0, s>>>(L, queries, L.max_depth + 2, leaf_min, seeds, nseed,
+                                 static_cast<int>(first), order, ctr);
+    if (kSome) return;
+  }
 }
 
 // Leaf rounds of the lanes, measured: at half the live lanes for booleans, three
@@ -1104,8 +1117,10 @@ hipError_t launch_mesh_shape_collide(const MeshShapeLaunch& in, int waves, hipSt
     MS_TRY(mem.get(&queries, static_cast<size_t>(L.num_queries)));
     meshshape_setup<<<static_cast<unsigned>((L.num_queries + kBlk - 1) / kBlk), kBlk, 0, s>>>(
         L, queries);
-    auto descent =
-        waves == 1 ? launch_descent<1> : (waves == 3 ? launch_descent<3> : launch_descent<2>);
+    auto descent = order ? launch_descent<2, true>
+                         : (waves == 1 ? launch_descent<1, false>
+                                       : (waves == 3 ? launch_descent<3, false>
+                                                     : launch_descent<2, false>));
     descent(L, queries, seeds, ctr, order, kinds, s);
   }
   MS_TRY(hipGetLastError());

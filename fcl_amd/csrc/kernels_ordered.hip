@@ -14,7 +14,7 @@
 // query, up to 2,353 dependent visits where the mean is 287.  Measured,
 // 2 x 2,420 triangles: 10,000 queries to their first contact 3.5 ms with a
 // lane per query, 0.21 ms with a wavefront; 4,096 queries to 8 contacts with
-// geometry 9.4 -> 0.26 ms; one collide() call 440 -> 140 us.
+// geometry 9.4 -> 0.26 ms; one collide() call 440 -> 72 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -164,6 +164,10 @@ __device__ __forceinline__ void write_records(const CollideLaunch& L, const Quer
   }
 }
 
+// Statistics: none, summed in 32 bits per list entry, and the same where the
+// entries' sums could outgrow them (ord_audit).
+enum : int { kNoCounts = 0, kCounts32 = 1, kAuditedCounts = 2 };
+
 template <int G, bool kStats, bool kContact>
 struct OrderedWave {
   static constexpr int kGroups = kWave / G;
@@ -180,10 +184,11 @@ struct OrderedWave {
 // wavefront looks through `chunk` queries at a time for the others.  (With
 // statistics the lists of four quarters leave LDS for three wavefronts per
 // SIMD.)
-template <int G, bool kStats, bool kContact, bool kSome>
-__global__ void __launch_bounds__(kWave, G == 16 && kStats ? 3 : 4)
+template <int G, int kCounts, bool kContact, bool kSome>
+__global__ void __launch_bounds__(kWave, G == 16 && kCounts != kNoCounts ? 3 : 4)
     collide_ordered(CollideLaunch L, int margin, int leaf_min, int chunk) {
   constexpr int kCap = list_cap<G>();
+  constexpr bool kStats = kCounts != kNoCounts;
   __shared__ OrderedWave<G, kStats, kContact> W;
   const LaneGroup<G> g;
   const int gi = g.first / G;
@@ -263,7 +268,7 @@ __global__ void __launch_bounds__(kWave, G == 16 && kStats ? 3 : 4)
     if (__ballot(q != -2) == 0) break;
     // the window: lane k holds the list's entry k from the top
     int n = q >= 0 ? ord_window<G, kCap>(T.sp, margin) : 0;
-    if constexpr (kStats)
+    if constexpr (kCounts == kAuditedCounts)
       if (__ballot(--T.audit_in < 0) != 0) ord_audit(g, S, T, L.carry_max, n);
     const bool on = g.lane < n;
     unsigned long long e = 0;
@@ -355,17 +360,27 @@ hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStr
     if (e != hipSuccess || L.lanes_max == kAllLanes) return e;
   }
   const int margin = stack_need + 2;
-  const bool stats = L.bv_tests || L.leaf_tests;
+  // (statistics that fit 32 bits by the meshes' sizes need no audits, which
+  // take 1 % of a single call)
+  const int counts = !(L.bv_tests || L.leaf_tests)
+                         ? kNoCounts
+                         : (L.node_pairs_max <= static_cast<long long>(L.carry_max) ? kCounts32
+                                                                                     : kAuditedCounts);
   // (a quarter's list must hold a tree path and a step)
   const bool narrow = L.num_queries >= kNarrowMin && L.cap == 1 && margin + 16 <= list_cap<16>();
   const int G = narrow ? 16 : kWave;
   auto pick = [&](auto g, auto some) {
     constexpr int kG = decltype(g)::value;
     constexpr bool kSome = decltype(some)::value;
-    return L.contact ? (stats ? collide_ordered<kG, true, true, kSome>
-                              : collide_ordered<kG, false, true, kSome>)
-                     : (stats ? collide_ordered<kG, true, false, kSome>
-                              : collide_ordered<kG, false, false, kSome>);
+    if (counts == kNoCounts)
+      return L.contact ? collide_ordered<kG, kNoCounts, true, kSome>
+                       : collide_ordered<kG, kNoCounts, false, kSome>;
+    if constexpr (!kSome)
+      if (counts == kCounts32)
+        return L.contact ? collide_ordered<kG, kCounts32, true, kSome>
+                         : collide_ordered<kG, kCounts32, false, kSome>;
+    return L.contact ? collide_ordered<kG, kAuditedCounts, true, kSome>
+                     : collide_ordered<kG, kAuditedCounts, false, kSome>;
   };
   const std::integral_constant<int, 16> quarter;
   const std::integral_constant<int, 64> whole;
