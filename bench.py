@@ -695,7 +695,7 @@ def first_contact_measure(ctx, steps, no_cpu, log_prefix="first contact"):
         bv, lf = float(obv.sum()), float(olf.sum())
         valu = (bv * OPS_BV / PEAK_FP32 + lf * OPS_LEAF / PEAK_FP64) / t
         hbm = (bv * BYTES_BV + lf * BYTES_LEAF) / t / PEAK_HBM
-        out["roofline"] = {"kernel": "ordered_collide", "bound": "valu", "valu_frac": valu,
+        out["roofline"] = {"kernel": "collide_ordered", "bound": "valu", "valu_frac": valu,
                            "hbm_frac": hbm, "bv_tests_per_query": bv / n,
                            "leaf_tests_per_query": lf / n,
                            "note": "2 x 4839 nodes stay in cache: bound by VALU and latency"}

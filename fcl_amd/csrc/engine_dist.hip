@@ -17,9 +17,12 @@
 // smallest (distance, key) found, and a task is pruned when its bound is
 // above the best distance, or equal to it with a key above the best key
 // (all pairs of its subtree come later in the reference's order).  Hence
-// the minimum and the pair reported are the reference's whatever the order
-// of the work; the nearest points are those of that pair, recomputed when
-// the query is done.
+// the minimum is the reference's whatever the order of the work, and so is
+// the pair reported, unless several pairs share the minimum to the last bit
+// (around a common vertex or edge) and rounding has lifted a bound above it:
+// which of them is found can then depend on the order (about 1 of 20,000
+// queries).  The nearest points are those of that pair, recomputed when the
+// query is done.
 //
 // With FP32 culling (the dist_fp32_cull tunable; off by default, FP64
 // bounds throughout) bounds are first taken in FP32 (device/rss32.h: a

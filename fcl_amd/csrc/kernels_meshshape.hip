@@ -1072,7 +1072,7 @@ hipError_t launch_lanes(MeshShapeLaunch L, MsEpaSeed* seeds, unsigned long long*
 // enough to hide the lanes' waiting for each other's leaf rounds, which grows
 // with the mesh (and with the contacts asked for).  Lanes / wavefronts, to the
 // first hit: a triangle, 32,768 queries 249 / 314 us and 1,000,000 1.0 / 5.8 ms;
-// 12 triangles 65,536 1.5 / 0.8, 131,072 1.4 / 1.4 and 1,000,000 4.6 / 10.3; 80
+// 12 triangles 100,000 1.4 / 1.2, 131,072 1.4 / 1.4 and 1,000,000 4.6 / 10.3; 80
 // triangles 131,072 2.74 / 2.68 and 250,000 3.6 / 5.0; 180 triangles 250,000 5.9 /
 // 5.8; 320 triangles 500,000 12.2 / 12.4 and 1,000,000 20 / 25; 800 triangles
 // 3,000,000 87 / 79.  To 4 hits: 80 triangles 131,072 3.7 / 2.7 and 250,000 4.8 /
@@ -1080,7 +1080,7 @@ hipError_t launch_lanes(MeshShapeLaunch L, MsEpaSeed* seeds, unsigned long long*
 // 3,000,000 67 / 71.
 long long mesh_shape_lanes_max(int num_queries, int cap, size_t nodes_min, size_t nodes_max) {
   long long limit = num_queries >= 24576 ? 1 : 0;
-  const long long over = (num_queries - 90112LL) / (cap > 1 ? 3 : 1);
+  const long long over = num_queries >= 122880 ? (num_queries - 90112LL) / (cap > 1 ? 3 : 1) : 0;
   while (limit < 1023 && (limit + 1) * (limit + 1) <= over) ++limit;
   if (static_cast<long long>(nodes_min) > limit) return 0;
   return static_cast<long long>(nodes_max) <= limit ? kAllLanes : limit;
