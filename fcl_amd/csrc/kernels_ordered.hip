@@ -41,12 +41,16 @@ constexpr int list_cap() {
 // wavefront: the chip is full either way, and a group of 16 tests less ahead
 // of a query's answer.  1,000,000 queries of 2 x 2,420 triangles 15.5 ms by
 // whole wavefronts, 8.7 ms by quarters; 10,000 queries 0.23 against 0.37 ms.
-// With statistics 65,536 queries 1.31 against 1.21 and 250,000 4.7 against
-// 3.6 ms, with geometry 1.37 against 1.02 and 5.0 against 3.1 (2 x 80
-// triangles, 1,000,000: 11.7 against 6.9 and 13.1 against 6.9).  With more
-// contacts little is tested in vain, and whole wavefronts stay ahead (100,000
-// queries, 8 contacts: 2.3 against 3.9 ms).
+// With statistics 65,536 queries 1.31 against 1.17 and 1,000,000 18.4 against
+// 12.7 ms, with geometry 1.38 against 1.02 and 19.8 against 11.0 (2 x 80
+// triangles, 1,000,000: 11.7 against 6.9 and 13.1 against 6.9); but between 2 x
+// 20,480 triangles, where the batch waits for its heaviest queries, 65,536 3.9
+// against 12.2 and 3.5 against 8.9 (1,000,000: 39 against 54 and 38 against 40),
+// so both only below kNarrowPairs node pairs.  With more contacts little is
+// tested in vain, and whole wavefronts stay ahead (100,000 queries, 8 contacts:
+// 2.3 against 3.9 ms).
 constexpr int kNarrowMin = 65536;
+constexpr long long kNarrowPairs = 1LL << 26;  // 2 x 4,096 triangles
 
 // The FP64 test of a node pair the cull left unsure.
 __device__ __forceinline__ bool overlap64(const QueryXf64& x, const ObbNode64* n1,
@@ -367,7 +371,8 @@ hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStr
                          : (L.node_pairs_max <= static_cast<long long>(L.carry_max) ? kCounts32
                                                                                      : kAuditedCounts);
   // (a quarter's list must hold a tree path and a step)
-  const bool narrow = L.num_queries >= kNarrowMin && L.cap == 1 && margin + 16 <= list_cap<16>();
+  const bool narrow = L.num_queries >= kNarrowMin && L.cap == 1 && margin + 16 <= list_cap<16>() &&
+                      ((counts == kNoCounts && !L.contact) || L.node_pairs_max <= kNarrowPairs);
   const int G = narrow ? 16 : kWave;
   auto pick = [&](auto g, auto some) {
     constexpr int kG = decltype(g)::value;
@@ -388,8 +393,11 @@ hipError_t launch_collide_ordered(const CollideLaunch& L, int stack_need, hipStr
   const std::false_type all;
   auto kernel = L.lanes_max > 0 ? (narrow ? pick(quarter, some) : pick(whole, some))
                                 : (narrow ? pick(quarter, all) : pick(whole, all));
-  // a wavefront's queries to look through: few enough to leave all busy
-  const int chunk = L.lanes_max > 0 ? std::min(std::max(L.num_queries / 8192, 1), kWave) : kWave / G;
+  // A wavefront's queries to look through: few, as it answers its heavy ones one
+  // after the other (a box against 20,480 triangles with statistics, 250,000
+  // queries: 5.0 ms in 8,192 parts, 4.1 in 65,536, 4.0 where no query is light)
+  const int chunk =
+      L.lanes_max > 0 ? std::min(std::max(L.num_queries / 131072, kWave / G), kWave) : kWave / G;
   kernel<<<group_blocks((L.num_queries + chunk - 1LL) / chunk), kWave, 0, s>>>(
       L, margin, narrow ? 8 : 16, chunk);
   return hipGetLastError();
